@@ -152,15 +152,16 @@ __global__ __launch_bounds__(kRThreads * CW) void q8r_gemv_kc_kernel(const int8_
   }
 }
 
-// The T-wide form (T > 1): the same per-output arithmetic, with each weight
-// load serving many positions. A workgroup takes 8 rows x up to kRTPW
-// positions; per chunk of K its lanes load their leaves' blocks once (CVT:
-// codes widened to fp32 once, for up to 2 blocks per leaf), then the
-// positions' x of that chunk are staged in LDS tp at a time (bf16 widened to
-// fp32, 36-float padded blocks) and every position runs the leaf chains and
-// the tree of the single-position kernel. The chunk partials of a (position,
-// row) go to an LDS running sum in chunk order, y = ((0 + p_0) + p_1) + ...
-constexpr int kRTPW = 32;      // positions per workgroup
+// The T-wide form for a few positions (more run on the matrix cores,
+// q8r_gemm.hip): the same per-output arithmetic, with each weight load serving
+// all positions. A workgroup takes 8 rows x up to kRTPW positions; per chunk
+// of K its lanes load their leaves' blocks once (CVT: codes widened to fp32
+// once, for up to 2 blocks per leaf), then the positions' x of that chunk are
+// staged in LDS tp at a time (bf16 widened to fp32, 36-float padded blocks) and
+// every position runs the leaf chains and the tree of the single-position
+// kernel. The chunk partials of a (position, row) go to an LDS running sum in
+// chunk order, y = ((0 + p_0) + p_1) + ...
+constexpr int kRTPW = 8;       // positions per workgroup
 
 template <int BPL, bool CVT>
 __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__restrict__ codes,
@@ -279,10 +280,15 @@ extern "C" int pq_q8r_gemv(const int8_t *codes, const float *scales, const uint1
   const int yb = y_dtype == PQ_DTYPE_BF16 ? 1 : 0;
   hipStream_t st = as_stream(stream);
   static const int env_t = env_int("PQ_Q8R_POSWISE");   // 1: one position per workgroup row at any T
-  if (T > 1 && env_t != 1) {   // the T-wide form: each weight load serves up to 32 positions
+  if (T > 1 && env_t != 1) {   // each weight load serves many positions
+    // The matrix cores pad T to 16 or 32 positions; below that the vector
+    // kernel costs by the position. Per launch, vector / matrix: 2048 x 2048 at
+    // 8 positions 8.3 / 9.0 us, 16384 x 2048 22.5 / 22.3, at 12 positions 512 x
+    // 2048 10.6 / 8.6; with over 2 blocks a leaf (codes widened per use, 4.4 us
+    // a position at 2048 x 7680) at 4 positions 17.4 / 24.3, at 8 30.9 / 24.7.
+    if (T > (bpl <= 2 ? 8 : 5)) return q8r_mfma(codes, scales, x, y, yb, N, K, T, st);
     // positions per LDS tile: as many 36-float padded chunks as fit 18 KB, at most 8 (small tiles keep
-    // several workgroups per CU: a 256-token prompt through 24 layers of hidden 2048 / FFN 8192 takes
-    // 41 ms with 72 KB tiles, 25 ms with 18 KB)
+    // several workgroups per CU: 18 KB measured faster than 72 KB)
     const size_t per = (size_t)(KC / kQ) * kRXStride * sizeof(float);
     static const int env_kb = env_int("PQ_Q8R_TILE_KB");
     const size_t budget = (size_t)(env_kb > 0 ? env_kb : 18) * 1024;

@@ -17,6 +17,10 @@ constexpr int kRMaxChunks = 8;   // 2048-wide chunks a row may hold in the chunk
 
 __host__ __device__ inline int q8r_chunk(int K) { return (K >= 2048 && K % 2048 == 0) ? 2048 : K; }
 
+// The many-position form on the fp32 matrix cores (q8r_gemm.hip); yb: bf16 y.
+int q8r_mfma(const int8_t *codes, const float *scales, const uint16_t *x, void *y, int yb, int N, int K, int T,
+             hipStream_t st);
+
 struct RBlocks {
   v4i c[2 * 8];
   float s[8];

@@ -195,3 +195,48 @@ def test_q8r_gemv_fused_embed(pq, dev, K):
         torch.cuda.synchronize()
         assert torch.equal(xo, row), tok
         assert torch.equal(y.view(torch.int16), want.view(torch.int16)), tok
+
+
+# The matrix-core form (more than 8 positions; 5 with over 2 blocks a leaf):
+# 16- and 32-wide tiles at their edges (one row or position more or less than
+# a tile), ragged leaves (65 and 9 blocks a chunk, one block, a class without
+# blocks), several chunks.
+@pytest.mark.parametrize("N,K,T", [(1, 32, 9), (15, 288, 16), (17, 2080, 17), (31, 2048, 33), (33, 4096, 31),
+                                   (64, 7680, 6), (16, 8160, 12), (40, 8192, 9), (2100, 256, 65), (520, 6144, 129)])
+def test_q8r_matrix_tiles(orc, pq, dev, N, K, T):
+    print(f"q8r matrix N={N} K={K} T={T}", flush=True)
+    W, S, xb = _case(orc, N, K, T, SEED + 3 * N + K, signed_scales=True)
+    want = orc.q8r_gemm(W, S, xb)
+    y = _run(pq, dev, W, S, xb, pq.DT_F32).cpu().numpy()
+    assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
+
+
+def test_q8r_matrix_exponents(orc, pq, dev):
+    """x over the whole exponent range: sums that round at every step, subnormal products and sums, overflow."""
+    N, K, T = 70, 2048, 40
+    W, S, xb = _case(orc, N, K, T, SEED + 77, signed_scales=True)
+    e = orc.gen_codes(SEED + 78, T * K).reshape(T, K).astype(np.int32)
+    e[: T // 4] //= 8                       # +-15: every step rounds
+    e[T // 4: T // 2] = -127 + e[T // 4: T // 2] // 16   # subnormal
+    e[T // 2: 3 * T // 4] = 120             # overflow to infinity and NaN
+    x = np.ldexp(orc.bf2f(xb).astype(np.float64), e)
+    with np.errstate(over="ignore"):
+        xb = orc.f2bf(np.clip(x, -3e38, 3e38).astype(np.float32))
+    want = orc.q8r_gemm(W, S, xb)
+    y = _run(pq, dev, W, S, xb, pq.DT_F32).cpu().numpy()
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(y), nan)
+    assert np.array_equal(y.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+
+
+@pytest.mark.parametrize("N,K,T", [(16416, 512, 96), (8200, 1024, 40)])
+def test_q8r_matrix_matches_few_positions(pq, dev, N, K, T):
+    """More tiles than workgroups: the same bits as the vector kernel's, 8 positions at a time."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(N + K)
+    W = torch.randint(-127, 128, (N, K), dtype=torch.int8, device=dev, generator=g)
+    S = torch.rand((N, K // 32), device=dev, generator=g) * 0.02
+    x = torch.randn((T, K), device=dev, generator=g).to(torch.bfloat16)
+    y = pq.q8r_gemv(W, S, x, out_dtype=pq.DT_F32)
+    want = torch.cat([pq.q8r_gemv(W, S, x[t:t + 8], out_dtype=pq.DT_F32) for t in range(0, T, 8)])
+    assert torch.equal(y.view(torch.int32), want.view(torch.int32))
