@@ -58,6 +58,14 @@ int attn_decode_dev(const uint16_t *q, int q_stride, const uint16_t *kcache, con
                     const int32_t *pos_dev, int ctx, int nh, int nkv, int hd, float scale, int win, void *ws,
                     size_t ws_bytes, hipStream_t st);
 
+// pq_qlow_gemm on the fp32 matrix cores (qlow_gemm.hip) in tiles of mt = 16 or
+// 32 rows x positions; yb: bf16 y, ks: the order's K slices (2 or 4).
+// qlow_mfma_tile: the tile to take, or 0 for the vector kernel (rv rounds of
+// 256 workgroups of rs rows x tb positions).
+int qlow_mfma_tile(int N, int K, int T, int ks, long long rv, int rs, int tb);
+int qlow_mfma(int mt, const uint8_t *pc, const uint32_t *ps, const uint16_t *x, void *y, int yb, int N, int K, int T,
+              int ldy, int bits, int ks, hipStream_t st);
+
 // pq_argmax_parts that also appends the id: ids[ctr[0]++] = id, ctr[1]++.
 int argmax_parts_step(const float *parts, int nparts, int32_t *out, int32_t *ids, int32_t *ctr, hipStream_t st);
 

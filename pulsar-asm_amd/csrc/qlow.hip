@@ -29,6 +29,7 @@
 // exactly (v_fma_mix_f32).
 #include "pq_device.h"
 #include "pq_host.h"
+#include "pq_internal.h"
 #include "q8_common.h"
 #include "pq_prologue.h"
 
@@ -426,7 +427,8 @@ __global__ __launch_bounds__(NT) void qlow_gemv_kernel(const uint8_t *__restrict
 }
 
 // ---------------------------------------------------------- T positions
-// The GEMV of TB positions per workgroup, one position block per blockIdx.y
+// (Few positions, or few rows: qlow_mfma_tile sends the rest to the matrix
+// cores, qlow_gemm.hip.) The GEMV of TB positions per workgroup, one position block per blockIdx.y
 // (a prompt's low-bit linears, which the reference runs one position at a
 // time): every position's arithmetic is the single-position kernel's, in the
 // same order, so y[t] equals pq_qlow_gemv of x[t] bit for bit. A group's codes
@@ -916,6 +918,10 @@ extern "C" int pq_qlow_gemm(const uint8_t *pcodes, const uint16_t *pscales, cons
              "pq_qlow_gemm: packed codes and x must be 16-byte aligned");
   int RS, TB;
   qlow_gemm_shape(N, K, T, RS, TB);
+  const long long rv = ((long long)(N / RS) * ((T + TB - 1) / TB) + 255) / 256;
+  if (const int mt = qlow_mfma_tile(N, K, T, qlow_ks(K), rv, RS, TB))
+    return qlow_mfma(mt, pcodes, reinterpret_cast<const uint32_t *>(pscales), x, y, y_dtype == PQ_DTYPE_BF16 ? 1 : 0,
+                     N, K, T, ldy, bits, qlow_ks(K), as_stream(stream));
   const int G = K / kQ, XL = (K / 8 + kQgNT - 1) / kQgNT;
   const size_t lds = qlow_gemm_lds(G, RS, TB);
   PQ_REQUIRE(lds <= kMaxLds && TB * XL <= 8, PQ_ERR_ARG, "pq_qlow_gemm: K=%d exceeds the workgroup's LDS", K);

@@ -213,3 +213,48 @@ def test_qlow_gemm_equals_gemv(orc, pq, dev, bits, N, K, T):
         for t in range(T):
             xb = X[t].view(torch.int16).cpu().numpy().view(np.uint16)
             assert np.array_equal(y[t].cpu().numpy().view(np.uint32), orc.qlow_gemv(Q, S, xb).view(np.uint32))
+
+
+# The matrix-core forms at their edges, row by row the bits of the one-position
+# GEMV: 16-wide tiles (one position past a tile, a last tile of one; slices of
+# 34 groups, not a multiple of the 4 taken at once; an odd number of row tiles)
+# and 32-wide ones (2 and 4 slices, ragged positions), at both widths of code.
+# K = 16384 is the longest row.
+@pytest.mark.parametrize("bits,N,K,T", [(5, 2048, 4352, 33), (4, 2080, 2048, 65), (5, 4128, 512, 49), (4, 1024, 16384, 65),
+                                        (4, 16384, 256, 64), (5, 16416, 256, 97), (5, 4096, 4352, 255), (4, 4096, 4096, 256)])
+def test_qlow_matrix_tiles(pq, dev, bits, N, K, T):
+    print(f"qlow matrix bits={bits} N={N} K={K} T={T}", flush=True)
+    g = torch.Generator(device=dev)
+    g.manual_seed(N + K + T + bits)
+    Q = torch.randint(0, 1 << bits, (N, K), dtype=torch.uint8, device=dev, generator=g)
+    S = (torch.randn((N, K // 32, 2), device=dev, generator=g) * 0.05).half()
+    w = pq.QlowWeight(Q, S, bits)
+    X = (torch.randn((T, K), device=dev, generator=g) * 2.0).to(torch.bfloat16)
+    X[T - 1] *= 1e30                                  # rounding at other exponents
+    X[T - 2] *= 1e-38                                 # subnormal products and sums
+    wide = torch.full((T, N + 24), float("nan"), dtype=torch.float32, device=dev)
+    pq.qlow_gemm(w, X, out_dtype=pq.DT_F32, out=wide[:, :N])
+    yb = pq.qlow_gemm(w, X)
+    for t in sorted({0, 1, 15, 16, T // 2, T - 2, T - 1}):
+        assert torch.equal(wide[t, :N].view(torch.int32), pq.qlow_gemv(w, X[t], out_dtype=pq.DT_F32).view(torch.int32)), t
+        assert torch.equal(yb[t].view(torch.int16), pq.qlow_gemv(w, X[t]).view(torch.int16)), t
+    assert torch.isnan(wide[:, N:]).all()
+    first = pq.qlow_gemm(w, X[:2], out_dtype=pq.DT_F32)   # the vector form
+    assert torch.equal(first.view(torch.int32), wide[:2, :N].contiguous().view(torch.int32))
+
+
+def test_qlow_matrix_infinity(pq, dev):
+    """An infinite or NaN x reaches its own position's outputs only."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(5)
+    w = pq.QlowWeight(torch.randint(0, 16, (4096, 2048), dtype=torch.uint8, device=dev, generator=g),
+                      (torch.randn((4096, 64, 2), device=dev, generator=g) * 0.05).half(), 4)
+    X = torch.randn((40, 2048), device=dev, generator=g).to(torch.bfloat16)
+    want = pq.qlow_gemm(w, X, out_dtype=pq.DT_F32)
+    X[7, 100], X[33, 2047] = float("inf"), float("nan")
+    y = pq.qlow_gemm(w, X, out_dtype=pq.DT_F32)
+    keep = [t for t in range(40) if t not in (7, 33)]
+    assert torch.equal(y[keep].view(torch.int32), want[keep].view(torch.int32))
+    for t in (7, 33):
+        one = pq.qlow_gemv(w, X[t], out_dtype=pq.DT_F32)
+        assert torch.equal(torch.isnan(y[t]), torch.isnan(one)) and not torch.isfinite(y[t]).any()
