@@ -4,9 +4,12 @@ Each wrapper validates shapes and dtypes on the host, calls one C entry point
 on torch's current stream and raises PQError with the library's message on a
 negative return code.
 """
+import ctypes as C
+
 import torch
 
 from . import check, lib
+from ._abi import GemvPrologue
 
 __all__ = ["stream_ptr", "Q8Weight", "q8_quant", "q8_gemv", "q8_gemm", "q8r_gemv", "q8r_gemv_fused", "QlowWeight", "qlow_gemv", "qlow_gemv_fused", "qlow_gemv_fused_swiglu", "qlow_gemm", "DT_F32", "DT_BF16", "rmsnorm", "qk_prep", "qk_prep_ref", "attn_ref", "attn_decode_ref", "attn_decode_ref_q8gate",
            "attn_decode", "conv", "silu_mul", "argmax", "embed", "q8k_quant", "tq2_gemv", "tq2_gemv_batch", "gemv_fused",
@@ -21,7 +24,11 @@ DT_BF16 = 1
 
 
 def stream_ptr():
-    return torch.cuda.current_stream().cuda_stream
+    """torch's current stream on the current device, as the C ABI takes it. Read without the
+    Stream object that torch.cuda.current_stream() builds around it on each call."""
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t):
@@ -65,21 +72,21 @@ class Q8Weight:
 
 def q8_quant(x):
     """x [T][K] fp32 or bf16 -> (qx int8 [T][K], dx fp32 [T][K/32])."""
-    squeeze = x.dim() == 1
-    x2 = x.reshape(1, -1) if squeeze else x
-    T, K = x2.shape
-    x2 = x2.contiguous()
-    qx = torch.empty((T, K), dtype=torch.int8, device=x.device)
-    dx = torch.empty((T, K // 32), dtype=torch.float32, device=x.device)
-    L = lib()
-    if x2.dtype == torch.float32:
-        rc = L.pq_q8_quant_f32(x2.data_ptr(), qx.data_ptr(), dx.data_ptr(), K, T, stream_ptr())
-    elif x2.dtype in (torch.bfloat16, torch.int16, torch.uint16):
-        rc = L.pq_q8_quant_bf16(x2.data_ptr(), qx.data_ptr(), dx.data_ptr(), K, T, stream_ptr())
+    shape = x.shape
+    T, K = (1, shape[0]) if len(shape) == 1 else shape
+    if not x.is_contiguous():
+        x = x.contiguous()
+    lead, dev = shape[:-1], x.device
+    qx = torch.empty(shape, dtype=torch.int8, device=dev)
+    dx = torch.empty((*lead, K // 32), dtype=torch.float32, device=dev)
+    if x.dtype == torch.float32:
+        fn = lib().pq_q8_quant_f32
+    elif x.dtype in (torch.bfloat16, torch.int16, torch.uint16):
+        fn = lib().pq_q8_quant_bf16
     else:
         raise ValueError("x must be fp32 or bf16")
-    check(rc, "pq_q8_quant")
-    return (qx[0], dx[0]) if squeeze else (qx, dx)
+    check(fn(x.data_ptr(), qx.data_ptr(), dx.data_ptr(), K, T, stream_ptr()), "pq_q8_quant")
+    return qx, dx
 
 
 def q8_gemv(w, qx, dx, out_dtype=DT_F32, out=None):
@@ -195,7 +202,6 @@ def qlow_gemm(w, x, out_dtype=DT_BF16, out=None):
 def qlow_gemv_fused(w, kind, out_dtype=DT_BF16, out=None, eps=1e-5, **ptrs):
     """The Q4/Q5 GEMV at T = 1 with x from a prologue (pq_qlow_gemv_fused):
     kind RESNORM, NORM, SILU or CONV, ptrs as for gemv_fused."""
-    import ctypes as C
     p = _prologue(kind, eps, ptrs)
     if out is None:
         out = torch.empty(w.N, dtype=torch.float32 if out_dtype == DT_F32 else torch.bfloat16, device=w.pcodes.device)
@@ -208,7 +214,6 @@ def qlow_gemv_fused_swiglu(w, kind, out=None, eps=1e-5, **ptrs):
     """The FFN's gate/up GEMV on a low-bit [gate | up] tensor (w.N = 2F rows)
     with a RESNORM or NORM prologue and the SwiGLU epilogue
     (pq_qlow_gemv_fused_swiglu): bf16 [F] = silu(gate) * up."""
-    import ctypes as C
     p = _prologue(kind, eps, ptrs)
     F = w.N // 2
     if out is None:
@@ -321,11 +326,13 @@ def embed(w, tokens, H, vocab):
 # ------------------------------------------------------------- ternary path
 def q8k_quant(x):
     """x fp32 [T][K] -> Q8_K blocks, uint8 [T][K/256*292]."""
-    x2 = x.reshape(1, -1) if x.dim() == 1 else x
-    T, K = x2.shape
-    out = torch.empty((T, K // 256 * 292), dtype=torch.uint8, device=x.device)
-    check(lib().pq_q8k_quant(x2.contiguous().data_ptr(), out.data_ptr(), K, T, stream_ptr()), "pq_q8k_quant")
-    return out[0] if x.dim() == 1 else out
+    shape = x.shape
+    T, K = (1, shape[0]) if len(shape) == 1 else shape
+    if not x.is_contiguous():
+        x = x.contiguous()
+    out = torch.empty((*shape[:-1], K // 256 * 292), dtype=torch.uint8, device=x.device)
+    check(lib().pq_q8k_quant(x.data_ptr(), out.data_ptr(), K, T, stream_ptr()), "pq_q8k_quant")
+    return out
 
 
 def tq2_gemv(codes, scales, xq, K, N, out=None):
@@ -341,7 +348,6 @@ def tq2_gemv(codes, scales, xq, K, N, out=None):
 def tq2_gemv_batch(tensors, xq, K, outs=None):
     """1..3 ternary tensors [(codes, scales), ...] of one K over the same Q8_K
     xq in one launch (pq_tq2_gemv_batch) -> [y fp32 [N_i], ...]."""
-    import ctypes as C
     n = len(tensors)
     rows = [int(c.shape[0]) for c, _ in tensors]
     if outs is None:
@@ -356,7 +362,6 @@ def tq2_gemv_batch(tensors, xq, K, outs=None):
 
 # ------------------------------------------------------- fused decode path
 def _prologue(kind, eps, ptrs):
-    from ._abi import GemvPrologue
     p = GemvPrologue()
     p.kind = kind
     p.eps = eps
@@ -376,7 +381,6 @@ def gemv_fused(w, kind, out_dtype=DT_BF16, out=None, parts=None, eps=1e-5, **ptr
     """GEMV whose input x is produced by a prologue (pq_q8_gemv_fused). ptrs are
     tensors for the pq_gemv_prologue fields (qx, dx, h, x_in, x_out, w0, w1, gu,
     bcx, ring_in, ring_out, taps, emb (a Q8Weight), tok) plus ints ntaps, vocab."""
-    import ctypes as C
     p = _prologue(kind, eps, ptrs)
     if out is None:
         out = torch.empty(w.N, dtype=torch.float32 if out_dtype == DT_F32 else torch.bfloat16, device=w.pcodes.device)
@@ -390,7 +394,6 @@ def q8r_gemv_fused(codes, scales, kind, out_dtype=DT_BF16, out=None, parts=None,
     at T = 1 with x from a prologue (pq_q8r_gemv_fused): kind RESNORM, NORM,
     SILU or CONV, ptrs as for gemv_fused; parts (fp32, 2 * pq_q8r_gemv_parts(N))
     receives the per-workgroup argmax pairs."""
-    import ctypes as C
     N, K = codes.shape
     if scales.shape != (N, K // 32) or scales.dtype != torch.float32:
         raise ValueError("scales must be fp32 [N][K/32]")
@@ -406,7 +409,6 @@ def q8r_gemv_fused_swiglu(codes, scales, kind, out=None, eps=1e-5, **ptrs):
     """The reference-numerics gate/up GEMV (codes int8 [2F][K]: gate rows, then
     up rows) with a RESNORM or NORM prologue and the silu(gate) * up epilogue
     (pq_q8r_gemv_fused_swiglu): returns y bf16 [F]."""
-    import ctypes as C
     N, K = codes.shape
     if scales.shape != (N, K // 32) or scales.dtype != torch.float32:
         raise ValueError("scales must be fp32 [N][K/32]")
@@ -421,7 +423,6 @@ def q8r_gemv_fused_swiglu(codes, scales, kind, out=None, eps=1e-5, **ptrs):
 def gemv_fused_swiglu(w, kind, eps=1e-5, **ptrs):
     """gate/up GEMV (w packed with gate_up=True) with prologue `kind` and the
     silu(gate)*up epilogue: returns the Q8_0 row (qx int8 [F], dx fp32 [F/32])."""
-    import ctypes as C
     if not getattr(w, "gate_up", False):
         raise ValueError("gemv_fused_swiglu needs a Q8Weight packed with gate_up=True")
     p = _prologue(kind, eps, ptrs)
