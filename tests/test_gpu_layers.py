@@ -116,6 +116,48 @@ def test_attention(orc, pq, dev, npos_last, T, nh, nkv, hd, win):
     assert np.array_equal(qx.cpu().numpy(), orc.q8_quant_bf16(want)[0])
 
 
+# Many queries (the matrix tiles) equal the one-query calls bit for bit: GQA
+# groups 1, 2, 4 and 8, head_dim 64 and 128, chunks that end inside a split and
+# inside a tile, windows (rows whose keys begin inside a split or that see none
+# of it), a q row stride that no 16-byte load fits, and keys whose masked V is
+# infinite or NaN (a row must not see it).
+@pytest.mark.parametrize("nh,nkv,hd,pos0,T,win,pad,bad", [
+    (32, 8, 64, 0, 301, 0, 0, False), (32, 8, 64, 1500, 33, 0, 1, False), (8, 8, 64, 70, 517, 0, 0, True),
+    (16, 8, 64, 300, 210, 100, 0, True), (16, 4, 128, 0, 403, 0, 3, True), (16, 4, 128, 777, 269, 256, 0, True),
+    (8, 1, 128, 5, 700, 0, 0, False), (8, 1, 128, 900, 450, 256, 0, False), (32, 8, 64, 0, 400, 1, 0, True)])
+def test_attention_many_queries(pq, dev, nh, nkv, hd, pos0, T, win, pad, bad):
+    print(f"attn tiles {nh}/{nkv}x{hd} pos0={pos0} T={T} win={win}", flush=True)
+    g = torch.Generator(device=dev)
+    g.manual_seed(T + pos0 + hd)
+    n, kvd, qs = pos0 + T, nkv * hd, nh * hd + pad
+    q = (torch.randn((T, qs), device=dev, generator=g) * 2).to(torch.bfloat16)
+    kc = (torch.randn((n + 5, kvd), device=dev, generator=g) * 2).half()
+    vc = (torch.randn((n + 5, kvd), device=dev, generator=g) * 5).half()
+    kc[n:], vc[n:] = float("nan"), float("nan")   # past the chunk: never read
+    hot = []
+    if bad:
+        hot = [pos0 + T // 2, pos0 + T - 1]
+        vc[hot[0], ::3], vc[hot[1], 1::2] = float("inf"), float("nan")
+    gate = (torch.randn((T, nh), device=dev, generator=g) * 3).to(torch.bfloat16)
+    out = torch.zeros((T, nh * hd), dtype=torch.bfloat16, device=dev)
+    qx = torch.empty((T, nh * hd), dtype=torch.int8, device=dev)
+    dx = torch.empty((T, nh * hd // 32), dtype=torch.float32, device=dev)
+    pq.attn_decode(q, qs, kc, vc, pos0, nh, nkv, hd, T, 0.125, gate=gate, gate_stride=nh, out=out, out_stride=nh * hd,
+                   qx=qx, dx=dx, win=win)
+    for t in sorted({0, 1, 7, 31, T // 3, T // 2 - 1, T // 2, T // 2 + 1, 3 * T // 4, T - 2, T - 1}):
+        one = torch.zeros(nh * hd, dtype=torch.bfloat16, device=dev)
+        q1, d1 = torch.empty_like(qx[0]), torch.empty_like(dx[0])
+        pq.attn_decode(q[t], qs, kc, vc, pos0 + t, nh, nkv, hd, 1, 0.125, gate=gate[t], gate_stride=nh, out=one,
+                       out_stride=nh * hd, qx=q1, dx=d1, win=win)
+        nan = torch.isnan(one)
+        assert torch.equal(torch.isnan(out[t]), nan), t
+        assert torch.equal(out[t][~nan].view(torch.int16), one[~nan].view(torch.int16)), t
+        seen = [p for p in hot if p <= pos0 + t and (win == 0 or p > pos0 + t - win)]
+        assert torch.isfinite(one).all() == (not seen), t
+        if not seen:
+            assert torch.equal(qx[t], q1) and torch.equal(dx[t].view(torch.int32), d1.view(torch.int32)), t
+
+
 def test_qk_prep_ref_bf16_cache(orc, pq, dev):
     """pq_qk_prep_ref: q as pq_qk_prep leaves it, and the cache rows the bf16 k
     (normed, rotated) and v as they are (k_kv_write's copy)."""
