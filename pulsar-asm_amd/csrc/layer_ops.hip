@@ -27,13 +27,9 @@ __device__ __forceinline__ void quant_store(const float *v, int8_t *qx, float *d
   for (int o = 1; o < 32 / E; o <<= 1) a = fmaxf(a, __shfl_xor(a, o, 64));
   const float d = a / 127.0f;
   int8_t q[E];
-  const float dd = d != 0.0f ? d : 1.0f;   // d = 0: the block is all zero (q = 0), no branch
+  const Q8Div dv(d);   // the block's one divisor
 #pragma unroll
-  for (int i = 0; i < E; i++) {
-    int t = (int)__builtin_rintf(v[i] / dd);
-    t = t > 127 ? 127 : (t < -127 ? -127 : t);
-    q[i] = (int8_t)t;
-  }
+  for (int i = 0; i < E; i++) q[i] = (int8_t)q8_code(dv.div(v[i]));
 #pragma unroll
   for (int i = 0; i < E; i++) qx[e0 + i] = q[i];
   if ((e0 & 31) == 0) dx[e0 >> 5] = d;
@@ -89,7 +85,8 @@ __global__ __launch_bounds__(1024) void rmsnorm_kernel(uint16_t *__restrict__ x,
 }
 
 // ------------------------------------------------- q/k norm, RoPE, KV write
-// One wave per (head, position); lane l holds dimensions l + 64e, e < HD/64
+// One wave per (head, position), 4 heads a workgroup (one wave each was bound
+// by the launch of 24576 workgroups at 512 positions); lane l holds dimensions l + 64e, e < HD/64
 // (HD = 64 or 128). Heads [0, nh) are q (norm + rope, in place), [nh, nh+nkv)
 // k (norm + rope, then written to the fp16 cache), [nh+nkv, nh+2nkv) v
 // (written to the cache). The sum of squares is k_headnorm's (head_sumsq).
@@ -99,13 +96,15 @@ __global__ __launch_bounds__(1024) void rmsnorm_kernel(uint16_t *__restrict__ x,
 // cache holds the bf16 values as the reference's k_kv_write copies them
 // (157-162); else fp16 of them.
 template <int HD, bool KVB>
-__global__ __launch_bounds__(64) void qk_prep_kernel(uint16_t *__restrict__ qkv, int row_stride,
+__global__ __launch_bounds__(256) void qk_prep_kernel(uint16_t *__restrict__ qkv, int row_stride,
                                                       const float *__restrict__ qn, const float *__restrict__ kn,
                                                       const float *__restrict__ cs, uint16_t *__restrict__ kc,
                                                       uint16_t *__restrict__ vc, int pos0, int nh, int nkv, int rot,
                                                       float eps, const int32_t *__restrict__ pos_dev) {
   constexpr int E = HD / 64;
-  const int head = blockIdx.x, t = blockIdx.y, l = threadIdx.x;
+  const int head = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.y;
+  const int l = threadIdx.x & 63;
+  if (head >= nh + 2 * nkv) return;
   const int pos = (pos_dev != nullptr ? *pos_dev : pos0) + t;
   uint16_t *row = qkv + (size_t)t * row_stride;
   const int kvd = nkv * HD;
@@ -225,12 +224,15 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t *__restric
   const int e0 = (blockIdx.x * blockDim.x + threadIdx.x) * E;
   const uint16_t *g = gu + t * 2 * F + (IL ? 32 * (e0 / 32) : 0);
   const uint16_t *u = IL ? g + 32 : g + F;
+  uint16_t gv[E], uv[E];   // loaded whole before e^x branches: 2 loads a thread, not 2 E
+  __builtin_memcpy(gv, g + e0, sizeof gv);
+  __builtin_memcpy(uv, u + e0, sizeof uv);
   float o[E];
 #pragma unroll
   for (int i = 0; i < E; i++) {
-    const float a = bf2f(g[e0 + i]);
+    const float a = bf2f(gv[i]);
     const float sg = 1.0f / (1.0f + expf_pq(-a));
-    o[i] = bf2f(f2bf((a * sg) * bf2f(u[e0 + i])));
+    o[i] = bf2f(f2bf((a * sg) * bf2f(uv[i])));
   }
   if (y != nullptr) {
 #pragma unroll
@@ -242,17 +244,24 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t *__restric
 // ------------------------------------------------------------------ argmax
 // The pick of k_argmax (am_better: the largest value above kAmFloor, ties in
 // its thread-slot order; -1 when there is none), by any tree: a scan per
-// thread, then the wave butterfly and the waves in order.
+// thread, then the wave butterfly and the waves in order. A thread's indices
+// lie in one slot of k_argmax's 256 and ascend, so its first strict maximum is
+// its pick. One workgroup; kAmLoads values a thread load together (one a step,
+// each waited for, took 50 us for 128000 values).
+constexpr int kAmLoads = 16;
+
 __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ v, int n, int32_t *__restrict__ out) {
   __shared__ float bv[16];
   __shared__ int bi[16];
   float best = kAmFloor;
   int idx = -1;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    float cv;
-    int ci;
-    am_leaf(v[i], i, cv, ci);
-    if (am_better(cv, ci, best, idx)) { best = cv; idx = ci; }
+  for (unsigned i0 = threadIdx.x; i0 < (unsigned)n; i0 += kAmLoads * 1024) {
+    float c[kAmLoads];
+#pragma unroll
+    for (int k = 0; k < kAmLoads; k++) c[k] = i0 + k * 1024 < (unsigned)n ? v[i0 + k * 1024] : kAmFloor;
+#pragma unroll
+    for (int k = 0; k < kAmLoads; k++)
+      if (c[k] > best) { best = c[k]; idx = (int)(i0 + k * 1024); }
   }
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -363,7 +372,7 @@ int qk_prep_launch(uint16_t *qkv, int row_stride, const float *q_norm, const flo
                    uint16_t *kcache, uint16_t *vcache, int pos0, const int32_t *pos_dev, int nh, int nkv, int hd,
                    int rot, int T, float eps, hipStream_t st, bool kv_bf16) {
 #define PQ_QKP(HH, KB)                                                                                             \
-  launch(qk_prep_kernel<HH, KB>, dim3(nh + 2 * nkv, T), dim3(64), 0, st, qkv, row_stride, q_norm, k_norm, rope_cs, \
+  launch(qk_prep_kernel<HH, KB>, dim3((nh + 2 * nkv + 3) / 4, T), dim3(256), 0, st, qkv, row_stride, q_norm, k_norm, rope_cs, \
          kcache, vcache, pos0, nh, nkv, rot, eps, pos_dev)
   if (hd == 64) {
     if (kv_bf16) PQ_QKP(64, true);
