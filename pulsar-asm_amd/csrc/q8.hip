@@ -485,7 +485,7 @@ __global__ __launch_bounds__(kGemmThreads) void q8_gemm_kernel(const int8_t *__r
     }
 }
 
-// The tile-parallel form (small and mid-sized N): a workgroup = S 32-row
+// The tile-parallel form (one position block): a workgroup = S 32-row
 // slices x 32 positions, 8*S waves; wave w takes slice w % S and chunk
 // 8*rd + w / S of round rd, so a round's 8 chunks of every slice load at once.
 // Per round the 32 positions' activations (2048 K) and dx are loaded first,
@@ -495,14 +495,12 @@ __global__ __launch_bounds__(kGemmThreads) void q8_gemm_kernel(const int8_t *__r
 // for two workgroups per CU). Same numerics as the walking form.
 // PH = 16 gives a workgroup 16 positions (the A operand's other 16 rows read
 // zeros and their outputs are neither folded nor written): twice the
-// workgroups and half the fold per wave, for GEMMs with few slices. AUX is the
-// weight loads' cache policy: nontemporal, or cached where many position
-// blocks' workgroups re-read the same weights.
+// workgroups and half the fold per wave, for GEMMs with few slices.
 constexpr int kTileSlots = 8;
 constexpr size_t kTileActBytes = 32 * (size_t)kGemmARow;
 constexpr size_t kTileLds = kTileActBytes + (size_t)kTileSlots * kCB * 32 * 4;
 
-template <int S, bool PIPE, int PH = 32, int AUX = kAuxNT>
+template <int S, bool PIPE, int PH = 32>
 __global__ __launch_bounds__(64 * kTileSlots * S) void q8_gemm_tile_kernel(const int8_t *__restrict__ pc,
                                                                         const uint16_t *__restrict__ ps,
                                                                         const int8_t *__restrict__ qx,
@@ -560,7 +558,7 @@ __global__ __launch_bounds__(64 * kTileSlots * S) void q8_gemm_tile_kernel(const
     v4i wv[kCB];
     const int oc = valid ? c * kCB * kSlab + (h * kTR + jt) * 16 : kRsrcOob;
 #pragma unroll
-    for (int i = 0; i < kCB; i++) wv[i] = __builtin_amdgcn_raw_buffer_load_b128(rc, oc + i * kSlab, 0, AUX);
+    for (int i = 0; i < kCB; i++) wv[i] = __builtin_amdgcn_raw_buffer_load_b128(rc, oc + i * kSlab, 0, kAuxNT);
     const v4i sv = __builtin_amdgcn_raw_buffer_load_b128(rs, valid ? (c * kTR + jt) * 16 : kRsrcOob, 0, 0);
     if (rd > 0) lds_barrier();   // the previous round's fold reads of the partials are done
 #pragma unroll
@@ -606,6 +604,167 @@ __global__ __launch_bounds__(64 * kTileSlots * S) void q8_gemm_tile_kernel(const
       if (y_bf16) reinterpret_cast<uint16_t *>(y)[(size_t)pos * N + row] = f2bf(yv[k]);
       else reinterpret_cast<float *>(y)[(size_t)pos * N + row] = yv[k];
     }
+  }
+}
+
+// The chunk-parallel form (many positions): a workgroup = S waves on one tile of
+// 64 rows x 32 positions, wave w taking chunks w, w + S, ... of K; a round's S
+// chunk partials then fold into y through LDS in chunk order, as the order adds
+// them. Each wave stages the 256 bytes of its chunk's 32 positions (whole lines
+// from global memory, loaded a round ahead) and their dx in LDS of its own, so
+// waves meet only for the fold; the partials reuse that LDS.
+//
+// What bounds it: the fold's 3 vector instructions per output and block (48 per
+// 32 x 32 x 32 MFMA, 192 of its 32 matrix cycles), then the LDS reads of dx.
+// Two row slices per wave read the activations and dx once for both; slice 1's
+// MFMA runs under slice 0's fold and the next block's under slice 1's. A
+// block's weight registers take the next chunk's block as soon as its MFMA is
+// issued: one register set, loads a chunk ahead. Against 64-row tiles of 16
+// waves that staged 2048 K for all and folded unpipelined: 2048 x 8192 at 256
+// positions 28.3 -> 20.8 us, 3104 x 2048 at 512 31.5 -> 21.0 (310 TOP/s), 2048 x
+// 2048 at 64 7.5 -> 6.7.
+constexpr int kCkRow = kCB * kQ + 16;                          // padded LDS row of a position's chunk (bytes)
+constexpr int kCkWave = 32 * kCkRow + kCB * 32 * 4;            // a wave's LDS: activations, then dx [8][32]
+
+template <int S>
+__global__ __launch_bounds__(64 * S, 2) void q8_gemm_chunk_kernel(const int8_t *__restrict__ pc,
+                                                                   const uint16_t *__restrict__ ps,
+                                                                   const int8_t *__restrict__ qx,
+                                                                   const float *__restrict__ dx, void *__restrict__ y,
+                                                                   int y_bf16, int N, int K, int T, int npt) {
+  constexpr int NQ4 = 512 / (64 * S);   // float4s of the 64 x 32 outputs per thread
+  static_assert(kCkWave >= 2048 * 4, "a wave's partials reuse its LDS");
+  extern __shared__ __align__(16) unsigned char gsm[];
+  const int nb = K / kQ, nch = nchunks(K);
+  // workgroups go round-robin over the 8 XCDs: the position tiles of a row tile run on one XCD, whose L2 serves its
+  // weights again
+  const int idx = blockIdx.x >> 3, tile = (idx / npt) * 8 + (blockIdx.x & 7), t0 = (idx % npt) * 32;
+  if (tile * kTR >= N) return;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int h = lane >> 5, l32 = lane & 31;
+  unsigned char *mine = gsm + wave * kCkWave;
+  float *dxs = reinterpret_cast<float *>(mine + 32 * kCkRow);   // [8 blocks][32 positions]
+  const int np = T - t0 < 32 ? T - t0 : 32;
+  const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int8_t *>(pc + (size_t)tile * nb * kSlab), (short)0, nb * kSlab, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t *>(ps + (size_t)tile * nch * kTR * 8), (short)0, nch * kTR * 16, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(qx + (size_t)t0 * K), (short)0,
+                                                                      np * K, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(dx + (size_t)t0 * nb), (short)0, np * nb * 4, kRsrcWord3);
+  v4i av[8], dv, w[2][kCB], sv[2], sn[2];
+  auto act_load = [&](int c) {   // 4 positions of 16 pieces per load; the lane's position's dx of blocks 4h .. 4h + 3
+    const int col = c * kCB * kQ + (lane & 15) * 16;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      av[i] = __builtin_amdgcn_raw_buffer_load_b128(ra, c < nch && col < K ? (4 * i + (lane >> 4)) * K + col : kRsrcOob, 0, 0);
+    dv = __builtin_amdgcn_raw_buffer_load_b128(rd, c < nch ? (l32 * nb + c * kCB + 4 * h) * 4 : kRsrcOob, 0, 0);
+  };
+  auto act_store = [&]() {
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      *reinterpret_cast<v4i *>(mine + (4 * i + (lane >> 4)) * kCkRow + (lane & 15) * 16) = av[i];
+#pragma unroll
+    for (int k = 0; k < 4; k++) dxs[(4 * h + k) * 32 + l32] = __int_as_float(dv[k]);
+  };
+  auto w_off = [&](int c) { return c < nch ? c * kCB * kSlab + (h * kTR + l32) * 16 : kRsrcOob; };
+  auto s_load = [&](v4i *s, int c) {
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+      s[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, c < nch ? (c * kTR + 32 * u + l32) * 16 : kRsrcOob, 0, 0);
+  };
+  float a[2][16];
+  // One chunk of the wave into a; its weights are replaced by chunk cn's. FULL: 8 blocks (a chunk with fewer is the
+  // last one, and has no next).
+  auto chunk = [&](auto FULL, int nbc, int cn) {
+    constexpr bool full = decltype(FULL)::value;
+    const lds_ptr<v4i> ap = lds_base(reinterpret_cast<const v4i *>(mine + l32 * kCkRow + 16 * h));   // block i: ap[2 i]
+    const lds_ptr<f4v> dp = lds_base(reinterpret_cast<const f4v *>(dxs + 4 * h));   // block i, quad q: dp[8 i + 2 q]
+    const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const int on = w_off(cn);
+    v16i acc[2];
+    f4v d[4];   // block i's dx; quad q takes the next block's after its last use
+    v4i an = ap[0];
+#pragma unroll
+    for (int u = 0; u < 2; u++) acc[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(an, w[u][0], zero, 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 4; q++) d[q] = dp[2 * q];
+#pragma unroll
+    for (int i = 0; i < kCB; i++) {
+      if (!full && i >= nbc) break;
+      if (i + 1 < kCB) an = ap[2 * (i + 1)];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const float dw = half_of((uint32_t)sv[u][i >> 1], i & 1);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            a[u][4 * q + k] = __builtin_fmaf(dw * d[q][k], (float)acc[u][4 * q + k], a[u][4 * q + k]);
+          if (u == 1 && i + 1 < kCB) d[q] = dp[8 * (i + 1) + 2 * q];
+        }
+        if (full) w[u][i] = __builtin_amdgcn_raw_buffer_load_b128(rc, on + i * kSlab + u * 32 * 16, 0, 0);
+        if (i + 1 < kCB && (full || i + 1 < nbc))
+          acc[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(an, w[u][i + 1], zero, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  act_load(wave);
+  {
+    const int o = w_off(wave);
+#pragma unroll
+    for (int i = 0; i < kCB; i++)
+#pragma unroll
+      for (int u = 0; u < 2; u++) w[u][i] = __builtin_amdgcn_raw_buffer_load_b128(rc, o + i * kSlab + u * 32 * 16, 0, 0);
+    s_load(sv, wave);
+  }
+  f4v yv[NQ4];
+#pragma unroll
+  for (int k = 0; k < NQ4; k++) yv[k] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int rb = 0; rb < nch; rb += S) {
+    const int c = rb + wave, cn = c + S;
+    act_store();
+    act_load(cn);
+    s_load(sn, cn);
+    if (c < nch) {
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) a[u][r] = 0.0f;
+      const int nbc = nb - c * kCB;
+      if (nbc >= kCB) chunk(std::integral_constant<bool, true>{}, kCB, cn);
+      else chunk(std::integral_constant<bool, false>{}, nbc, cn);
+      f4v *pp = reinterpret_cast<f4v *>(mine) + lane;   // [u][q][lane]
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          pp[(4 * u + q) * 64] = f4v{a[u][4 * q], a[u][4 * q + 1], a[u][4 * q + 2], a[u][4 * q + 3]};
+    }
+    sv[0] = sn[0];
+    sv[1] = sn[1];
+    lds_barrier();
+    const int n = nch - rb < S ? nch - rb : S;
+#pragma unroll
+    for (int k = 0; k < NQ4; k++)
+#pragma unroll
+      for (int s = 0; s < S; s++)
+        if (s < n) yv[k] = yv[k] + reinterpret_cast<const f4v *>(gsm + s * kCkWave)[tid + k * 64 * S];
+    if (rb + S < nch) lds_barrier();   // the next round's activations overwrite the partials
+  }
+#pragma unroll
+  for (int k = 0; k < NQ4; k++) {
+    const int e = tid + k * 64 * S, l = e & 63, q = (e >> 6) & 3;
+    const int row = tile * kTR + (e >> 8) * 32 + (l & 31), p = 8 * q + 4 * (l >> 5);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (p + j < np && row < N) {
+        const size_t o = (size_t)(t0 + p + j) * N + row;
+        if (y_bf16) reinterpret_cast<uint16_t *>(y)[o] = f2bf(yv[k][j]);
+        else reinterpret_cast<float *>(y)[o] = yv[k][j];
+      }
   }
 }
 
@@ -723,19 +882,22 @@ static int gemm_splits(int N, int K, int T, bool have_ws) {
 }
 
 // Which form runs a T-wide GEMM: 1 = the walking form (persistent, split K
-// with a workspace), 2 = tile form over 64-row tiles, 3 = tile form over 32-row
-// slices. PQ_GEMM_FORM (1..3) overrides the choice.
-enum { kFormWalk = 1, kFormTile = 2, kFormSlice = 3 };
-// Measured on the LFM-style shapes (hidden 2048): 32-row slices win at one
-// position block with K <= 2048 (one round), the walking form for the LM head
-// and for deeper K at one position block (split over workgroups), 64-row
-// tiles for mid-sized N over many position blocks.
+// with a workspace), 2 = the chunk-parallel form over 64-row tiles, 3 = tile
+// form over 32-row slices. PQ_GEMM_FORM (1..3) overrides the choice.
+enum { kFormWalk = 1, kFormChunk = 2, kFormSlice = 3 };
+// Measured on the LFM-style shapes (hidden 2048): at one position block 32-row
+// slices win with K <= 2048 (one round), the walking form for the LM head and
+// for deeper K (split over workgroups); over several the chunk-parallel form,
+// but for long N, whose rows the walking form's resident workgroups reuse from
+// LDS: us, walking / chunk, 16384 x 2048 at 64 positions 26.2 / 13.6, at 96 43.3
+// / 20.4, at 128 20.9 / 26.2, at 256 36.3 / 46.5; 15360 x 2048 at 256 49.8 (64-row
+// tiles) / 40.3; 65536 x 2048 at 64 44.0 / 45.1, at 256 136 / 153.
 static int gemm_form(int N, int K, int T) {
   static const int env = env_int("PQ_GEMM_FORM");
   if (env >= kFormWalk && env <= kFormSlice) return env;
   if (N >= 32768) return kFormWalk;
   if (T <= 32) return K > kGemmSegK ? kFormWalk : kFormSlice;
-  return N >= 16384 ? kFormWalk : kFormTile;
+  return N >= 16384 && T > 96 ? kFormWalk : kFormChunk;
 }
 
 extern "C" size_t pq_q8_gemm_workspace_bytes(int N, int K, int T) {
@@ -764,14 +926,16 @@ extern "C" int pq_q8_gemm_ws(const int8_t *pcodes, const uint16_t *pscales, cons
   const int yb = y_dtype == PQ_DTYPE_BF16 ? 1 : 0;
   hipStream_t st = as_stream(stream);
   const int form = gemm_form(N, K, T);
-  if (form == kFormTile) {   // with 8+ position blocks the weights' re-reads are served from cache (measured)
-    const dim3 grid((unsigned)ntiles(N), 1, (unsigned)((T + 31) / 32));
-    if (grid.z >= 8)
-      launch(q8_gemm_tile_kernel<2, false, 32, 0>, grid, dim3(64 * kTileSlots * 2), kTileLds, st, pcodes, pscales, qx,
-             dx, y, yb, N, K, T);
+  if (form == kFormChunk) {
+    // 8 waves a tile (one workgroup per CU) while the tiles fit the CUs once, else 4 (two per CU). Measured, 4 / 8
+    // waves: 2048 x 8192 at 256 positions (256 tiles) 29.2 / 20.8 us, at 512 (512) 39.9 / 42.2; 6144 x 2048 at 64 (192)
+    // 8.8 / 6.9, at 96 (288) 11.6 / 12.5
+    const int npt = (T + 31) / 32;
+    const dim3 grid((unsigned)((ntiles(N) + 7) / 8 * 8 * npt));
+    if ((long long)ntiles(N) * npt <= 256)
+      launch(q8_gemm_chunk_kernel<8>, grid, dim3(512), 8 * kCkWave, st, pcodes, pscales, qx, dx, y, yb, N, K, T, npt);
     else
-      launch(q8_gemm_tile_kernel<2, false>, grid, dim3(64 * kTileSlots * 2), kTileLds, st, pcodes, pscales, qx, dx, y,
-             yb, N, K, T);
+      launch(q8_gemm_chunk_kernel<4>, grid, dim3(256), 4 * kCkWave, st, pcodes, pscales, qx, dx, y, yb, N, K, T, npt);
     return check_launch("pq_q8_gemm");
   }
   if (form == kFormSlice) {

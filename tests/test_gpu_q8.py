@@ -138,3 +138,19 @@ def test_gemm_bitexact(orc, pq, dev, N, K, T):
     for t in range(0, T, max(1, T // 4)):
         y1 = pq.q8_gemv(w, qx[t], dx[t], out_dtype=pq.DT_BF16)
         assert torch.equal(y1.view(torch.int16), yb[t].view(torch.int16))
+
+
+# The chunk-parallel form (more than 32 positions) at its edges: 4 and 8 waves a
+# tile, one row and one position past a tile, fewer chunks than waves, a last
+# chunk of 1, 7 and 8 blocks, several rounds of chunks.
+@pytest.mark.parametrize("N,K,T", [(1, 32, 33), (65, 224, 64), (64, 256, 65), (127, 2080, 100), (300, 4384, 40),
+                                   (16320, 288, 97), (2112, 2304, 300), (4160, 8192, 129), (520, 16384, 36)])
+def test_gemm_chunk_form(orc, pq, dev, N, K, T):
+    print(f"gemm chunks N={N} K={K} T={T}", flush=True)
+    W, S, w = _weights(orc, pq, dev, N, K, SEED + 7 * N + K)
+    x = orc.gen_normal(SEED + 5 * T + K, T * K).reshape(T, K)
+    qx_r, dx_r = orc.q8_quant(x)
+    qx, dx = pq.q8_quant(torch.from_numpy(x).to(dev))
+    y = pq.q8_gemm(w, qx, dx).cpu().numpy()
+    bad = np.argwhere(_bits(y) != _bits(orc.q8_gemm(W, S, qx_r, dx_r)))
+    assert bad.shape[0] == 0, f"{bad.shape[0]} cells differ, first {bad[:5].tolist()}"
