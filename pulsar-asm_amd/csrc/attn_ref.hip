@@ -9,9 +9,10 @@
 // block of 256 per head (blockIdx.y the chunk position). Threads 0..255 are
 // the reference's: its 8 warps of 32 are the 32-lane halves of waves 0-3
 // (lane = tid & 31, warp = tid >> 5), so every sum keeps its place. The scores
-// do not depend on which warp forms them, so all 32 warps of the 1024 threads
-// share them (a quarter of the key rounds, four waves a SIMD to hide latency):
-//   score p (warp p mod 32): lane l's chain s = fl(s + fl(q_d * k_d)) over its
+// do not depend on which warp forms them, so all warps of the workgroup share
+// them: 32 of 1024 threads (a quarter of the key rounds, four waves a SIMD to
+// hide latency), or 16 or 8 where many workgroups hide it for each other.
+//   score p (warp p mod the warps): lane l's chain s = fl(s + fl(q_d * k_d)) over its
 //     hd/32 dims from 0, the shfl_down tree over the 32 lanes, fl(s * scale);
 //   m = the largest score (a max: any order gives it);
 //   e_p = e^(s_p - m) by pq::expf_pq, the build's e^x, where the reference
@@ -78,7 +79,7 @@ __device__ __forceinline__ void kv_unpack(const typename KVPiece<E>::T &w, float
   }
 }
 
-constexpr int kArThreads = 1024;     // 32 warps for the scores; the first 256 are the reference's
+constexpr int kArThreads = 1024;     // of one or few queries: 32 warps for the scores; the first 256 are the reference's
 
 // The decode launch's own q/k prep (attn_ref_kernel<HD, true>): the inputs of
 // qk_prep_kernel for the token's q, k and v rows.
@@ -116,8 +117,8 @@ struct AttnGate {
 // kvn instead, as the last key of its score warp and of its value segment, so
 // every sum keeps the order of the unfused pair (pq_qk_prep_ref, then the
 // attention of this kernel without PREP).
-template <int HD, bool PREP, bool GQ>
-__global__ __launch_bounds__(kArThreads) void attn_ref_kernel(const uint16_t *__restrict__ q, int q_stride,
+template <int HD, bool PREP, bool GQ, int NT>
+__global__ __launch_bounds__(NT) void attn_ref_kernel(const uint16_t *__restrict__ q, int q_stride,
                                                         uint16_t *__restrict__ kc, uint16_t *__restrict__ vc,
                                                         const uint16_t *__restrict__ gate, int gate_stride,
                                                         uint16_t *__restrict__ out, int out_stride, int pos0,
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(kArThreads) void attn_ref_kernel(const uint16_t *__
   constexpr int E = HD / 32;
   using KT = typename KVPiece<E>::T;
   extern __shared__ __align__(16) float sl[];   // the window's scores, then their e
-  __shared__ float red[kArThreads / 64];
+  __shared__ float red[NT / 64 > 8 ? NT / 64 : 8];   // the waves' maxima, then the 8 reference warps' sums
   __shared__ float seg[8][HD];
   __shared__ float qs[PREP ? HD : 1];                      // PREP: the position's q
   __shared__ __align__(16) uint16_t kvn[PREP ? 2 * HD : 2];   // PREP: its bf16 k, then v
@@ -151,7 +152,7 @@ __global__ __launch_bounds__(kArThreads) void attn_ref_kernel(const uint16_t *__
   // fastest: 290 keys at 256 threads 7.8 us at 8 a round, 8.4 at 16, 10.5 at 64
   // (head_dim 64).
   constexpr int B = kArRound;
-  constexpr int W = kArThreads / 32;   // score warps
+  constexpr int W = NT / 32;   // score warps
   const int nks = np > wid ? (np - wid + W - 1) / W : 0;   // this warp's keys: lo + wid + W j
   const int nk = np > wid ? (np - wid + 7) / 8 : 0;        // segment wid's keys (wid < 8): lo + wid + 8 j
   auto ld = [&](__amdgpu_buffer_rsrc_t r, KT *w, int j0, int stride) {
@@ -289,13 +290,13 @@ __global__ __launch_bounds__(kArThreads) void attn_ref_kernel(const uint16_t *__
   if (wid < 8) ld(rv, wv, 0, 8);
   __syncthreads();
   float mx = -1e30f;
-  for (int i = tid; i < np; i += kArThreads) mx = fmaxf(mx, sl[i]);
+  for (int i = tid; i < np; i += NT) mx = fmaxf(mx, sl[i]);
   mx = wave_max(mx);
   if ((tid & 63) == 0) red[tid >> 6] = mx;
   __syncthreads();
   float m = red[0];
 #pragma unroll
-  for (int w = 1; w < kArThreads / 64; w++) m = fmaxf(m, red[w]);
+  for (int w = 1; w < NT / 64; w++) m = fmaxf(m, red[w]);
   __syncthreads();
   if constexpr (GQ) {   // the head's gate row on y (wave 8; y was written before two barriers)
     if (tid >= 512 && tid < 576) {
@@ -373,10 +374,27 @@ static int attn_ref_launch(const uint16_t *q, int q_stride, const uint16_t *kcac
   uint16_t *kc = const_cast<uint16_t *>(kcache), *vc = const_cast<uint16_t *>(vcache);
   const AttnPrep p = pp != nullptr ? *pp : AttnPrep{};
   const AttnGate g = gq != nullptr ? *gq : AttnGate{};
-#define PQ_AR(HH, PR, GG)                                                                                  \
-  launch(attn_ref_kernel<HH, PR, GG>, grid, block, lds, st, q, q_stride, kc, vc, gate, gate_stride, out, \
+  // Many workgroups: fewer threads each, so that a CU holds several and one's
+  // score, softmax and value phases (only 4 waves work on the last) run beside
+  // another's. Measured at 1024 / 512 / 256 threads: 16 heads of 128, 203 queries in a
+  // window of 256 (3248 workgroups) 44.3 / 36.0 / 34.3 us, 512 from 0 (8192) 128 /
+  // 97 / 90; 32 heads of 64, 512 from 0 209 / 157 / 143; 8 heads of 64, 64 from 1500
+  // (512) 32.9 / 32.1 / 33.0; 16 heads of 128, 16 from 1500 (256) 23.9 / 24.9 / 32.1.
+  const long long wgs = (long long)nh * T;
+  const int nt = pp != nullptr || wgs < 512 ? kArThreads : wgs < 1024 ? 512 : 256;
+#define PQ_ARN(HH, TT)                                                                                  \
+  launch(attn_ref_kernel<HH, false, false, TT>, grid, dim3(TT), lds, st, q, q_stride, kc, vc, gate, gate_stride, out, \
          out_stride, pos0, pos_dev, nh, nkv, scale, win, p, g)
-  if (hd == 64) {
+#define PQ_AR(HH, PR, GG)                                                                                  \
+  launch(attn_ref_kernel<HH, PR, GG, kArThreads>, grid, block, lds, st, q, q_stride, kc, vc, gate, gate_stride, out, \
+         out_stride, pos0, pos_dev, nh, nkv, scale, win, p, g)
+  if (nt == 256) {
+    if (hd == 64) PQ_ARN(64, 256);
+    else PQ_ARN(128, 256);
+  } else if (nt == 512) {
+    if (hd == 64) PQ_ARN(64, 512);
+    else PQ_ARN(128, 512);
+  } else if (hd == 64) {
     if (pp != nullptr && gq != nullptr) PQ_AR(64, true, true);
     else if (pp != nullptr) PQ_AR(64, true, false);
     else PQ_AR(64, false, false);
@@ -386,6 +404,7 @@ static int attn_ref_launch(const uint16_t *q, int q_stride, const uint16_t *kcac
     else PQ_AR(128, false, false);
   }
 #undef PQ_AR
+#undef PQ_ARN
   return check_launch(pp != nullptr ? "pq_attn_decode_ref" : "pq_attn_ref");
 }
 

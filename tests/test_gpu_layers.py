@@ -209,6 +209,26 @@ def test_attention_ref(orc, pq, dev, npos_last, T, nh, nkv, hd, win):
     assert bad.shape[0] == 0, f"{bad.shape[0]} differ, first {bad[:4].tolist()}"
 
 
+# The 512-thread form (512 .. 1023 workgroups) and the 256-thread one at both
+# head_dims, with windows, equal the one-query calls (1024 threads) bit for bit.
+@pytest.mark.parametrize("pos0,T,nh,nkv,hd,win", [(283, 17, 32, 8, 64, 0), (500, 33, 32, 8, 64, 100),
+                                                  (0, 60, 16, 4, 128, 0), (270, 70, 16, 4, 128, 256)])
+def test_attention_ref_thread_counts(pq, dev, pos0, T, nh, nkv, hd, win):
+    g = torch.Generator(device=dev)
+    g.manual_seed(pos0 + T)
+    n = pos0 + T
+    q = (torch.randn((T, nh * hd), device=dev, generator=g) * 2).to(torch.bfloat16)
+    kc, vc = ((torch.randn((n, nkv * hd), device=dev, generator=g) * s).to(torch.bfloat16) for s in (2, 5))
+    gate = torch.randn((T, nh), device=dev, generator=g).to(torch.bfloat16)
+    out = torch.zeros((T, nh * hd), dtype=torch.bfloat16, device=dev)
+    pq.attn_ref(q, nh * hd, kc, vc, pos0, nh, nkv, hd, T, 0.125, out, nh * hd, gate=gate, gate_stride=nh, win=win)
+    for t in range(T):
+        one = torch.zeros(nh * hd, dtype=torch.bfloat16, device=dev)
+        pq.attn_ref(q[t], nh * hd, kc, vc, pos0 + t, nh, nkv, hd, 1, 0.125, one, nh * hd, gate=gate[t], gate_stride=nh,
+                    win=win)
+        assert torch.equal(out[t].view(torch.int16), one.view(torch.int16)), t
+
+
 def test_attention_ref_segment_order(orc, pq, dev):
     """The value segments add pairwise (the oracle's hand-derived case: 0x3f81
     where a sequential sum gives 0x3f80), and no gate leaves the output as is."""
