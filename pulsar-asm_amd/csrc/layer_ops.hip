@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t *__restric
   const int e0 = (blockIdx.x * blockDim.x + threadIdx.x) * E;
   const uint16_t *g = gu + t * 2 * F + (IL ? 32 * (e0 / 32) : 0);
   const uint16_t *u = IL ? g + 32 : g + F;
-  uint16_t gv[E], uv[E];   // loaded whole before e^x branches: 2 loads a thread, not 2 E
+  uint16_t gv[E], uv[E];   // loaded whole: 2 loads a thread, not 2 E
   __builtin_memcpy(gv, g + e0, sizeof gv);
   __builtin_memcpy(uv, u + e0, sizeof uv);
   float o[E];

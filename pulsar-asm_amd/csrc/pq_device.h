@@ -94,12 +94,12 @@ __device__ __forceinline__ uint16_t f2h(float f) {
 
 // e^x with the build's one definition: Cody & Waite reduction
 // n = rint(x*log2 e), r = (x - n*ln2_hi) - n*ln2_lo, degree-7 Taylor
-// polynomial in Horner form, then two exact power-of-two factors so only the
-// last multiply rounds. Identical operation sequence on the host side.
+// polynomial in Horner form, then the power of two, whose multiply alone
+// rounds (a subnormal result, once). Identical values on the host side, which
+// scales by two exact factors and branches; here v_ldexp_f32 and selects, so
+// that independent calls interleave (2^32 inputs compared: the same bits, NaN
+// for NaN; 1.55x the rate of the branches).
 __device__ __forceinline__ float expf_pq(float x) {
-  if (x != x) return x;
-  if (x > 88.72283935546875f) return __builtin_inff();
-  if (x < -104.0f) return 0.0f;
   const float n = __builtin_rintf(x * 1.44269502162933349609375f);
   float r = __builtin_fmaf(n, -0.693145751953125f, x);
   r = __builtin_fmaf(n, -1.428606765330187045e-06f, r);
@@ -111,11 +111,9 @@ __device__ __forceinline__ float expf_pq(float x) {
   p = __builtin_fmaf(p, r, 0.5f);
   p = __builtin_fmaf(p, r, 1.0f);
   p = __builtin_fmaf(p, r, 1.0f);
-  const int ni = (int)n;
-  const int a = ni / 2, b = ni - a;
-  const float fa = __uint_as_float((uint32_t)(a + 127) << 23);
-  const float fb = __uint_as_float((uint32_t)(b + 127) << 23);
-  return (p * fa) * fb;
+  float y = __builtin_amdgcn_ldexpf(p, (int)n);
+  y = x > 88.72283935546875f ? __builtin_inff() : y;
+  return x < -104.0f ? 0.0f : y;
 }
 
 // Wave64 xor-butterfly reductions. After step k every aligned group of 2^k
