@@ -19,9 +19,8 @@
 //     calls CUDA's expf (not restated bit for bit); thread t sums e over
 //     p = t, t + 256, ... in order, the shfl_down tree per warp, the 8 warp
 //     sums by the tree of offsets 4, 2, 1; inv = 1 / sum;
-//   the value sum: warp g (segment g) accumulates fl(w_p * v_pd), w_p =
-//     fl(e_p * inv), over p = g, g + 8, ... in order for the lane's hd/32
-//     dims; out_d = bf16 of the 8 segments added pairwise.
+//   the value sum: segment g (the reference's warp g) accumulates fl(w_p * v_pd), w_p =
+//     fl(e_p * inv), over p = g, g + 8, ... in order for each dim; out_d = bf16 of the 8 segments added pairwise.
 // p counts from the window's first key lo (the reference's i and p). head_dim
 // 128 is the reference's (4 dims a lane); 64 takes 2.
 #include "pq_device.h"
@@ -144,24 +143,45 @@ __global__ __launch_bounds__(NT) void attn_ref_kernel(const uint16_t *__restrict
   const int nrow = PREP ? npos - 1 : npos;
   const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(kc, (short)0, nrow * kvd * 2, kRsrcWord3);
   const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(vc, (short)0, nrow * kvd * 2, kRsrcWord3);
-  // score warp w's keys: lo + w + 32j; value segment w's (w < 8): lo + w + 8j.
-  // Rounds of kArRound keys whose loads all go out before the round is
-  // computed; the first round of value rows is loaded before the softmax,
-  // which hides its latency. The kernel is bound by instruction latency, so
-  // short rounds (the fewest key slots issued past the window) measured
-  // fastest: 290 keys at 256 threads 7.8 us at 8 a round, 8.4 at 16, 10.5 at 64
-  // (head_dim 64).
+  // score warp w's keys: lo + w + W j, in rounds of 8 whose loads all go out
+  // before the round is computed. Value segment g's keys lo + g + 8j are read by
+  // a whole wave, EV dims a lane (waves 0..7, or 0..3 with two segments each), in
+  // rounds of BV keys: the first round's loads go out before the softmax, each
+  // further one's before the round before it is added. Short score rounds (the
+  // fewest key slots issued past the window) measured fastest: 290 keys at 256
+  // threads 7.8 us at 8 a round, 8.4 at 16, 10.5 at 64 (head_dim 64). With one
+  // round of values in flight, half a wave a segment, the value sums took 13.6 us
+  // of a decode launch's 24 at 1500 keys (head_dim 128) and the scores 8.5 of
+  // mostly tree steps; with the form here and the shared trees below the launch
+  // takes 17.5, and 203 queries in a window of 256 34.3 -> 26.5. (One dim a lane
+  // and 16 value waves: 23.7, and 83 for the 203 queries: four times the
+  // instructions.)
   constexpr int B = kArRound;
-  constexpr int W = NT / 32;   // score warps
+  constexpr int W = NT / 32;                        // score warps
+  constexpr int EV = HD / 64, NS = NT >= 512 ? 1 : 2, VW = 8 / NS;   // dims a lane, segments a wave, value waves
+  constexpr int BV = GQ || NS == 2 ? 8 : 16;
   const int nks = np > wid ? (np - wid + W - 1) / W : 0;   // this warp's keys: lo + wid + W j
-  const int nk = np > wid ? (np - wid + 7) / 8 : 0;        // segment wid's keys (wid < 8): lo + wid + 8 j
-  auto ld = [&](__amdgpu_buffer_rsrc_t r, KT *w, int j0, int stride) {
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), vd = (tid & 63) * EV;
+  const int npv = PREP ? np - 1 : np;                      // value keys in the cache
+  const int nvk = wave < VW && npv > wave ? (npv - wave + 7) / 8 : 0;   // the wave's rounds: its first segment is longest
+  auto ld = [&](KT *w, int j0) {
 #pragma unroll
     for (int b = 0; b < B; b++)
-      w[b] = kv_load<E>(r, (int)(((size_t)(lo + wid + stride * (j0 + b)) * kvd + kvo) * 2));
+      w[b] = kv_load<E>(rk, (int)(((size_t)(lo + wid + W * (j0 + b)) * kvd + kvo) * 2));
   };
-  KT wk[B], wv[B];
-  if (nks > 0) ld(rk, wk, 0, W);   // the first round's keys load during the prep
+  auto ldv = [&](uint32_t (*w)[BV], int j0) {
+#pragma unroll
+    for (int k = 0; k < NS; k++)
+#pragma unroll
+      for (int b = 0; b < BV; b++) {
+        const int off = (int)(((size_t)(lo + wave + VW * k + 8 * (j0 + b)) * kvd + (size_t)kvh * HD + vd) * 2);
+        if constexpr (EV == 2) w[k][b] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rv, off, 0, 0);
+        else w[k][b] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rv, off, 0, 0) << 16;
+      }
+  };
+  KT wk[B];
+  uint32_t va[NS][BV], vb[NS][BV];
+  if (nks > 0) ld(wk, 0);   // the first round's keys load during the prep
   float qv[E];
   float gy[8], gw[8];   // GQ, threads 256..511: 8 elements of the residual and of the norm weight
   RBlocks gB;           // GQ, wave 8: the head's gate row (leaf L: blocks L and L + 32)
@@ -248,7 +268,7 @@ __global__ __launch_bounds__(NT) void attn_ref_kernel(const uint16_t *__restrict
     for (int j = 0; j < E; j++) qv[j] = bf2f(q[(size_t)t * q_stride + (size_t)h * HD + lane * E + j]);
   }
   for (int j0 = 0; j0 < nks; j0 += B) {
-    if (j0 > 0) ld(rk, wk, j0, W);
+    if (j0 > 0) ld(wk, j0);
     float s[B];
 #pragma unroll
     for (int b = 0; b < B; b++) {
@@ -258,24 +278,25 @@ __global__ __launch_bounds__(NT) void attn_ref_kernel(const uint16_t *__restrict
 #pragma unroll
       for (int j = 0; j < E; j++) s[b] = s[b] + qv[j] * kf[j];
     }
-    // the trees of the round's keys step by step (independent chains side by side)
+    // The trees of the round's 8 keys together: each step leaves every lane one
+    // key's partial of two (the sum of a pair is the same from either lane), so
+    // the steps at 16, 8 and 4 halve the values to fold, and lane l ends with the
+    // total of key (l / 16) + 2 (l / 8 mod 2) + 4 (l / 4 mod 2), stored once.
+    float t[4];
 #pragma unroll
-    for (int b = 0; b < B; b++) s[b] = add_down<16>(s[b]);
-#pragma unroll
-    for (int b = 0; b < B; b++) s[b] = add_down<8>(s[b]);
-#pragma unroll
-    for (int b = 0; b < B; b++) s[b] = add_down<4>(s[b]);
-#pragma unroll
-    for (int b = 0; b < B; b++) s[b] = add_down<2>(s[b]);
-#pragma unroll
-    for (int b = 0; b < B; b++) s[b] = add_down<1>(s[b]);
-    if (lane == 0) {
-#pragma unroll
-      for (int b = 0; b < B; b++) {
-        const int i = wid + W * (j0 + b);
-        if (i < np) sl[i] = s[b] * scale;
-      }
+    for (int b = 0; b < 4; b++) {   // rows 2r / 2r + 1 of 16 lanes take key 2b / 2b + 1
+      const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[2 * b]), __float_as_uint(s[2 * b + 1]), false, false);
+      t[b] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     }
+    const bool l8 = (lane & 8) != 0, l4 = (lane & 4) != 0;
+#pragma unroll
+    for (int b = 0; b < 4; b++) t[b] = add_down<8>(t[b]);   // every lane takes part in the cross-lane sums
+    const float u0 = l8 ? t[1] : t[0], u1 = l8 ? t[3] : t[2];
+    const float w0 = add_down<4>(u0), w1 = u1 + dpp_f<0x124>(u1);   // with lane l + 4 (row_ror:12), l - 4 (row_ror:4)
+    const float u = l4 ? w1 : w0;
+    const float tot = add_down<1>(add_down<2>(u));
+    const int i = wid + W * (j0 + (lane >> 4) + (l8 ? 2 : 0) + (l4 ? 4 : 0));
+    if ((lane & 3) == 0 && i < np) sl[i] = tot * scale;
   }
   if constexpr (PREP) {   // the position's own key (read as zeros above), from kvn
     const int ws = (np - 1) % W;
@@ -287,7 +308,7 @@ __global__ __launch_bounds__(NT) void attn_ref_kernel(const uint16_t *__restrict
       if (wid == ws && lane == 0) sl[np - 1] = s * scale;
     }
   }
-  if (wid < 8) ld(rv, wv, 0, 8);
+  if (nvk > 0) ldv(va, 0);
   __syncthreads();
   float mx = -1e30f;
   for (int i = tid; i < np; i += NT) mx = fmaxf(mx, sl[i]);
@@ -316,39 +337,60 @@ __global__ __launch_bounds__(NT) void attn_ref_kernel(const uint16_t *__restrict
   }
   __syncthreads();
   const float inv = 1.0f / (((red[0] + red[4]) + (red[2] + red[6])) + ((red[1] + red[5]) + (red[3] + red[7])));
-  // the value sum of segment wid over keys wid, wid + 8, ... (from lo); PREP
-  // leaves the last key to the step after the loop
-  const int npv = PREP ? np - 1 : np;
-  float acc[E];
+  for (int i = tid; i < np; i += NT) sl[i] = sl[i] * inv;   // w_p
+  lds_barrier();
+  // the value sums; PREP leaves the last key to the step after the loop
+  float acc[NS][EV];
 #pragma unroll
-  for (int j = 0; j < E; j++) acc[j] = 0.0f;
-  for (int j0 = 0; j0 < (wid < 8 ? nk : 0); j0 += B) {
-    if (j0 > 0) ld(rv, wv, j0, 8);
-    // branch-free, so the round's weight reads from LDS go out together: keys
-    // past the window read a clamped slot and leave acc as it is (a select)
+  for (int k = 0; k < NS; k++)
 #pragma unroll
-    for (int b = 0; b < B; b++) {
-      const int i = wid + 8 * (j0 + b);
-      const float wt = sl[i < np ? i : np - 1] * inv;
-      float vf[E];
-      kv_unpack<E>(wv[b], vf);
+    for (int e = 0; e < EV; e++) acc[k][e] = 0.0f;
+  auto add = [&](int k, float wt, uint32_t v) {
+    acc[k][EV - 1] = acc[k][EV - 1] + wt * __uint_as_float(v & 0xffff0000u);
+    if constexpr (EV == 2) acc[k][0] = acc[k][0] + wt * __uint_as_float(v << 16);
+  };
+  auto values = [&](const uint32_t (*w)[BV], int j0) {
+    if (wave + VW * (NS - 1) + 8 * (j0 + BV - 1) < npv) {   // whole rounds: the weights' LDS reads go out together
+      float wt[NS][BV];
 #pragma unroll
-      for (int j = 0; j < E; j++) {
-        const float a = acc[j] + wt * vf[j];
-        acc[j] = i < npv ? a : acc[j];
+      for (int k = 0; k < NS; k++)
+#pragma unroll
+        for (int b = 0; b < BV; b++) wt[k][b] = sl[wave + VW * k + 8 * (j0 + b)];
+#pragma unroll
+      for (int b = 0; b < BV; b++)
+#pragma unroll
+        for (int k = 0; k < NS; k++) add(k, wt[k][b], w[k][b]);
+    } else {
+#pragma unroll
+      for (int b = 0; b < BV; b++)
+#pragma unroll
+        for (int k = 0; k < NS; k++) {
+          const int i = wave + VW * k + 8 * (j0 + b);
+          if (i < npv) add(k, sl[i], w[k][b]);   // uniform
+        }
+    }
+  };
+  for (int j0 = 0; j0 < nvk; j0 += 2 * BV) {
+    if (j0 + BV < nvk) ldv(vb, j0 + BV);
+    values(va, j0);
+    if (j0 + BV >= nvk) break;
+    if (j0 + 2 * BV < nvk) ldv(va, j0 + 2 * BV);
+    values(vb, j0 + BV);
+  }
+  if (wave < VW) {
+#pragma unroll
+    for (int k = 0; k < NS; k++) {
+      const int g = wave + VW * k;
+      if constexpr (PREP) {   // the position's own value row: its segment's last key
+        if (g == (np - 1) % 8) {
+          const float wt = sl[np - 1];
+#pragma unroll
+          for (int e = 0; e < EV; e++) acc[k][e] = acc[k][e] + wt * bf2f(kvn[HD + vd + e]);
+        }
       }
-    }
-  }
-  if constexpr (PREP) {   // the position's own value row: its segment's last key
-    if (wid == (np - 1) % 8) {
-      const float wt = sl[np - 1] * inv;
 #pragma unroll
-      for (int j = 0; j < E; j++) acc[j] = acc[j] + wt * __uint_as_float((uint32_t)kvn[HD + lane * E + j] << 16);
+      for (int e = 0; e < EV; e++) seg[g][vd + e] = acc[k][e];
     }
-  }
-  if (wid < 8) {
-#pragma unroll
-    for (int j = 0; j < E; j++) seg[wid][lane * E + j] = acc[j];
   }
   __syncthreads();
   if (tid < HD) {
@@ -375,9 +417,9 @@ static int attn_ref_launch(const uint16_t *q, int q_stride, const uint16_t *kcac
   const AttnPrep p = pp != nullptr ? *pp : AttnPrep{};
   const AttnGate g = gq != nullptr ? *gq : AttnGate{};
   // Many workgroups: fewer threads each, so that a CU holds several and one's
-  // score, softmax and value phases (only 4 waves work on the last) run beside
-  // another's. Measured at 1024 / 512 / 256 threads: 16 heads of 128, 203 queries in a
-  // window of 256 (3248 workgroups) 44.3 / 36.0 / 34.3 us, 512 from 0 (8192) 128 /
+  // score, softmax and value phases (8 waves at most work on the last) run beside
+  // another's. Measured at 1024 / 512 / 256 threads (with the value sums on 4 waves):
+  // 16 heads of 128, 203 queries in a window of 256 (3248 workgroups) 44.3 / 36.0 / 34.3 us, 512 from 0 (8192) 128 /
   // 97 / 90; 32 heads of 64, 512 from 0 209 / 157 / 143; 8 heads of 64, 64 from 1500
   // (512) 32.9 / 32.1 / 33.0; 16 heads of 128, 16 from 1500 (256) 23.9 / 24.9 / 32.1.
   const long long wgs = (long long)nh * T;
