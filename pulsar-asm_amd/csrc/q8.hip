@@ -626,6 +626,43 @@ __global__ __launch_bounds__(64 * kTileSlots * S) void q8_gemm_tile_kernel(const
 constexpr int kCkRow = kCB * kQ + 16;                          // padded LDS row of a position's chunk (bytes)
 constexpr int kCkWave = 32 * kCkRow + kCB * 32 * 4;            // a wave's LDS: activations, then dx [8][32]
 
+// One chunk of two 32-row slices x 32 positions into a; block i's activations at
+// ap[2 i], its dx of position quad q at dp[8 i + 2 q]. FULL: 8 blocks, and each
+// block's weight registers take the block at offset `on` (the next chunk's) once
+// its MFMA is issued; else nbc blocks (a row's last chunk, which has no next).
+template <bool FULL>
+__device__ __forceinline__ void chunk2(float (*a)[16], v4i (*w)[kCB], const v4i *sv, lds_ptr<v4i> ap, lds_ptr<f4v> dp,
+                                       __amdgpu_buffer_rsrc_t rc, int on, int nbc) {
+  const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  v16i acc[2];
+  f4v d[4];   // block i's dx; quad q takes the next block's after its last use
+  v4i an = ap[0];
+#pragma unroll
+  for (int u = 0; u < 2; u++) acc[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(an, w[u][0], zero, 0, 0, 0);
+#pragma unroll
+  for (int q = 0; q < 4; q++) d[q] = dp[2 * q];
+#pragma unroll
+  for (int i = 0; i < kCB; i++) {
+    if (!FULL && i >= nbc) break;
+    if (i + 1 < kCB) an = ap[2 * (i + 1)];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const float dw = half_of((uint32_t)sv[u][i >> 1], i & 1);
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          a[u][4 * q + k] = __builtin_fmaf(dw * d[q][k], (float)acc[u][4 * q + k], a[u][4 * q + k]);
+        if (u == 1 && i + 1 < kCB) d[q] = dp[8 * (i + 1) + 2 * q];
+      }
+      if (FULL) w[u][i] = __builtin_amdgcn_raw_buffer_load_b128(rc, on + i * kSlab + u * 32 * 16, 0, 0);
+      if (i + 1 < kCB && (FULL || i + 1 < nbc))
+        acc[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(an, w[u][i + 1], zero, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
 template <int S>
 __global__ __launch_bounds__(64 * S, 2) void q8_gemm_chunk_kernel(const int8_t *__restrict__ pc,
                                                                    const uint16_t *__restrict__ ps,
@@ -675,42 +712,8 @@ __global__ __launch_bounds__(64 * S, 2) void q8_gemm_chunk_kernel(const int8_t *
       s[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, c < nch ? (c * kTR + 32 * u + l32) * 16 : kRsrcOob, 0, 0);
   };
   float a[2][16];
-  // One chunk of the wave into a; its weights are replaced by chunk cn's. FULL: 8 blocks (a chunk with fewer is the
-  // last one, and has no next).
-  auto chunk = [&](auto FULL, int nbc, int cn) {
-    constexpr bool full = decltype(FULL)::value;
-    const lds_ptr<v4i> ap = lds_base(reinterpret_cast<const v4i *>(mine + l32 * kCkRow + 16 * h));   // block i: ap[2 i]
-    const lds_ptr<f4v> dp = lds_base(reinterpret_cast<const f4v *>(dxs + 4 * h));   // block i, quad q: dp[8 i + 2 q]
-    const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const int on = w_off(cn);
-    v16i acc[2];
-    f4v d[4];   // block i's dx; quad q takes the next block's after its last use
-    v4i an = ap[0];
-#pragma unroll
-    for (int u = 0; u < 2; u++) acc[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(an, w[u][0], zero, 0, 0, 0);
-#pragma unroll
-    for (int q = 0; q < 4; q++) d[q] = dp[2 * q];
-#pragma unroll
-    for (int i = 0; i < kCB; i++) {
-      if (!full && i >= nbc) break;
-      if (i + 1 < kCB) an = ap[2 * (i + 1)];
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const float dw = half_of((uint32_t)sv[u][i >> 1], i & 1);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-#pragma unroll
-          for (int k = 0; k < 4; k++)
-            a[u][4 * q + k] = __builtin_fmaf(dw * d[q][k], (float)acc[u][4 * q + k], a[u][4 * q + k]);
-          if (u == 1 && i + 1 < kCB) d[q] = dp[8 * (i + 1) + 2 * q];
-        }
-        if (full) w[u][i] = __builtin_amdgcn_raw_buffer_load_b128(rc, on + i * kSlab + u * 32 * 16, 0, 0);
-        if (i + 1 < kCB && (full || i + 1 < nbc))
-          acc[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(an, w[u][i + 1], zero, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-  };
+  const lds_ptr<v4i> ap = lds_base(reinterpret_cast<const v4i *>(mine + l32 * kCkRow + 16 * h));
+  const lds_ptr<f4v> dp = lds_base(reinterpret_cast<const f4v *>(dxs + 4 * h));
   act_load(wave);
   {
     const int o = w_off(wave);
@@ -734,8 +737,8 @@ __global__ __launch_bounds__(64 * S, 2) void q8_gemm_chunk_kernel(const int8_t *
 #pragma unroll
         for (int r = 0; r < 16; r++) a[u][r] = 0.0f;
       const int nbc = nb - c * kCB;
-      if (nbc >= kCB) chunk(std::integral_constant<bool, true>{}, kCB, cn);
-      else chunk(std::integral_constant<bool, false>{}, nbc, cn);
+      if (nbc >= kCB) chunk2<true>(a, w, sv, ap, dp, rc, w_off(cn), kCB);
+      else chunk2<false>(a, w, sv, ap, dp, rc, 0, nbc);
       f4v *pp = reinterpret_cast<f4v *>(mine) + lane;   // [u][q][lane]
 #pragma unroll
       for (int u = 0; u < 2; u++)
@@ -765,6 +768,122 @@ __global__ __launch_bounds__(64 * S, 2) void q8_gemm_chunk_kernel(const int8_t *
         if (y_bf16) reinterpret_cast<uint16_t *>(y)[o] = f2bf(yv[k][j]);
         else reinterpret_cast<float *>(y)[o] = yv[k][j];
       }
+  }
+}
+
+// The row-parallel form (long N, many positions): a workgroup = 8 waves, each a
+// 64-row tile of its own, on 32 positions; the activations of 2048 K are staged
+// once for the 8, and a wave walks its chunks with chunk2 and adds each to y in
+// registers, so nothing is exchanged and waves meet only at a new segment. K is
+// whole chunks (a last chunk of fewer blocks costs registers that spill).
+// Against the walking form, whose waves take 32 rows: half the LDS reads of dx and
+// of the activations per output (they and the fold's instructions bound both):
+// 16384 x 2048 at 256 positions 40.1 -> 32.3 us (532 TOP/s), 65536 139 -> 121.
+constexpr int kRwRows = 8 * kTR;
+
+__global__ __launch_bounds__(512, 2) void q8_gemm_rows_kernel(const int8_t *__restrict__ pc,
+                                                               const uint16_t *__restrict__ ps,
+                                                               const int8_t *__restrict__ qx,
+                                                               const float *__restrict__ dx, void *__restrict__ y,
+                                                               int y_bf16, int N, int K, int T, int npt) {
+  extern __shared__ __align__(16) unsigned char gsm[];
+  int8_t(*as)[kGemmARow] = reinterpret_cast<int8_t(*)[kGemmARow]>(gsm);              // [32 positions]
+  float(*dxs)[32] = reinterpret_cast<float(*)[32]>(gsm + 32 * kGemmARow);            // [64 blocks][32]
+  const int nb = K / kQ, nch = nchunks(K);
+  // the position blocks of a group of rows run on one XCD (workgroup id mod 8), whose L2 serves its weights again
+  const int idx = blockIdx.x >> 3, gr = (idx / npt) * 8 + (blockIdx.x & 7), t0 = (idx % npt) * 32;
+  if (gr * kRwRows >= N) return;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int h = lane >> 5, l32 = lane & 31;
+  const bool live = gr * kRwRows + wave * kTR < N;   // a wave past N reads zeros and writes nothing
+  const int tile = live ? gr * 8 + wave : 0;
+  const int np = T - t0 < 32 ? T - t0 : 32;
+  const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int8_t *>(pc + (size_t)tile * nb * kSlab), (short)0, live ? nb * kSlab : 0, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t *>(ps + (size_t)tile * nch * kTR * 8), (short)0, live ? nch * kTR * 16 : 0, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(qx + (size_t)t0 * K), (short)0,
+                                                                      np * K, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(dx + (size_t)t0 * nb), (short)0, np * nb * 4, kRsrcWord3);
+  auto w_off = [&](int c) { return c < nch ? c * kCB * kSlab + (h * kTR + l32) * 16 : kRsrcOob; };
+  auto s_load = [&](v4i *s, int c) {
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+      s[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, c < nch ? (c * kTR + 32 * u + l32) * 16 : kRsrcOob, 0, 0);
+  };
+  v4i w[2][kCB], sv[2], sn[2];
+  float a[2][16], yv[2][16];
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) yv[u][r] = 0.0f;
+  for (int c0 = 0; c0 < nch; c0 += kGemmSegChunks) {
+    // the segment's activations (32 rows x 128 pieces of 16 B) and dx
+    v4i av[8];
+    float dv[4];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int e = tid + i * 512, col = c0 * kCB * kQ + (e & 127) * 16;
+      av[i] = __builtin_amdgcn_raw_buffer_load_b128(ra, col < K ? (e >> 7) * K + col : kRsrcOob, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int e = tid + i * 512, b = c0 * kCB + (e & 63);
+      dv[i] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rd, b < nb ? ((e >> 6) * nb + b) * 4 : kRsrcOob, 0, 0));
+    }
+    if (c0 > 0) lds_barrier();   // every wave is done with the segment before
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int e = tid + i * 512;
+      *reinterpret_cast<v4i *>(&as[e >> 7][(e & 127) * 16]) = av[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int e = tid + i * 512;
+      dxs[e & 63][e >> 6] = dv[i];
+    }
+    if (c0 == 0) {
+#pragma unroll
+      for (int i = 0; i < kCB; i++)
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+          w[u][i] = __builtin_amdgcn_raw_buffer_load_b128(rc, w_off(0) + i * kSlab + u * 32 * 16, 0, 0);
+      s_load(sv, 0);
+    }
+    lds_barrier();
+    const int ce = nch - c0 < kGemmSegChunks ? nch - c0 : kGemmSegChunks;
+    for (int cs = 0; cs < ce; cs++) {
+      const int c = c0 + cs;
+      s_load(sn, c + 1);
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) a[u][r] = 0.0f;
+      const lds_ptr<v4i> ap = lds_base(reinterpret_cast<const v4i *>(&as[l32][cs * kCB * kQ + 16 * h]));
+      const lds_ptr<f4v> dp = lds_base(reinterpret_cast<const f4v *>(&dxs[cs * kCB][4 * h]));
+      chunk2<true>(a, w, sv, ap, dp, rc, w_off(c + 1), kCB);
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        sv[u] = sn[u];
+#pragma unroll
+        for (int r = 0; r < 16; r++) yv[u][r] = yv[u][r] + a[u][r];
+      }
+    }
+  }
+  if (!live) return;
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int row = tile * kTR + 32 * u + l32;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int p = 8 * (r >> 2) + 4 * h + (r & 3);
+      if (p < np && row < N) {
+        const size_t o = (size_t)(t0 + p) * N + row;
+        if (y_bf16) reinterpret_cast<uint16_t *>(y)[o] = f2bf(yv[u][r]);
+        else reinterpret_cast<float *>(y)[o] = yv[u][r];
+      }
+    }
   }
 }
 
@@ -883,21 +1002,30 @@ static int gemm_splits(int N, int K, int T, bool have_ws) {
 
 // Which form runs a T-wide GEMM: 1 = the walking form (persistent, split K
 // with a workspace), 2 = the chunk-parallel form over 64-row tiles, 3 = tile
-// form over 32-row slices. PQ_GEMM_FORM (1..3) overrides the choice.
-enum { kFormWalk = 1, kFormChunk = 2, kFormSlice = 3 };
-// Measured on the LFM-style shapes (hidden 2048): at one position block 32-row
-// slices win with K <= 2048 (one round), the walking form for the LM head and
-// for deeper K (split over workgroups); over several the chunk-parallel form,
-// but for long N, whose rows the walking form's resident workgroups reuse from
-// LDS: us, walking / chunk, 16384 x 2048 at 64 positions 26.2 / 13.6, at 96 43.3
-// / 20.4, at 128 20.9 / 26.2, at 256 36.3 / 46.5; 15360 x 2048 at 256 49.8 (64-row
-// tiles) / 40.3; 65536 x 2048 at 64 44.0 / 45.1, at 256 136 / 153.
+// form over 32-row slices, 4 = the row-parallel form. PQ_GEMM_FORM (1..4)
+// overrides the choice (4 where K is whole chunks).
+enum { kFormWalk = 1, kFormChunk = 2, kFormSlice = 3, kFormRows = 4 };
+// At one position block 32-row slices win with K <= 2048 (one round), the
+// walking form for the LM head and for deeper K (split over workgroups). Over
+// several, the least of three times per 2048 of K, in ns: a chunk-parallel tile's
+// share of the chip, the row-parallel form's rounds of 256 workgroups (a round's
+// waves are bound by their own chains when few, by the CU when all run), the
+// walking form's rounds where it would not split K. Measured, walking / chunk /
+// row (us, * taken): 16384 x 2048 at 64 positions 26.2 / 13.6* / 25.7, at 96 43.3 /
+// 20.4* / 26.4, at 128 20.9* / 26.2 / 27.0, at 256 40.1 / 46.5 / 32.3*; 15360 at 256 -
+// / 39.3 / 31.2*; 65536 at 64 46.2 / 45.1 / 36.7*, at 256 139 / 153 / 121*; 6144 at 512
+// - / 31.4 / 30.6*; 3104 at 512 - / 20.4* / 27.3.
 static int gemm_form(int N, int K, int T) {
   static const int env = env_int("PQ_GEMM_FORM");
-  if (env >= kFormWalk && env <= kFormSlice) return env;
-  if (N >= 32768) return kFormWalk;
-  if (T <= 32) return K > kGemmSegK ? kFormWalk : kFormSlice;
-  return N >= 16384 && T > 96 ? kFormWalk : kFormChunk;
+  if ((env >= kFormWalk && env <= kFormSlice) || (env == kFormRows && K % (kCB * kQ) == 0)) return env;
+  if (T <= 32) return N >= 32768 || K > kGemmSegK ? kFormWalk : kFormSlice;
+  const long long P = (T + 31) / 32;
+  const long long rows = (N + kRwRows - 1) / kRwRows * P, walk = (N + 255) / 256 * P;   // work items
+  const long long t_ck = 22 * P * ntiles(N);
+  const long long t_rw = K % (kCB * kQ) == 0 ? (rows + 255) / 256 * 24000 + rows * 8000 / 256 : t_ck + 1;
+  const long long t_wk = walk >= 256 && (K <= kGemmSegK || N >= 32768) ? (walk + 255) / 256 * 20500 : t_ck + 1;
+  if (t_ck <= t_rw && t_ck <= t_wk) return kFormChunk;
+  return t_rw < t_wk ? kFormRows : kFormWalk;
 }
 
 extern "C" size_t pq_q8_gemm_workspace_bytes(int N, int K, int T) {
@@ -926,6 +1054,12 @@ extern "C" int pq_q8_gemm_ws(const int8_t *pcodes, const uint16_t *pscales, cons
   const int yb = y_dtype == PQ_DTYPE_BF16 ? 1 : 0;
   hipStream_t st = as_stream(stream);
   const int form = gemm_form(N, K, T);
+  if (form == kFormRows) {
+    const int npt = (T + 31) / 32, ngr = (N + kRwRows - 1) / kRwRows;
+    launch(q8_gemm_rows_kernel, dim3((unsigned)((ngr + 7) / 8 * 8 * npt)), dim3(512), kGemmLds, st, pcodes, pscales, qx, dx,
+           y, yb, N, K, T, npt);
+    return check_launch("pq_q8_gemm");
+  }
   if (form == kFormChunk) {
     // 8 waves a tile (one workgroup per CU) while the tiles fit the CUs once, else 4 (two per CU). Measured, 4 / 8
     // waves: 2048 x 8192 at 256 positions (256 tiles) 29.2 / 20.8 us, at 512 (512) 39.9 / 42.2; 6144 x 2048 at 64 (192)

@@ -154,3 +154,18 @@ def test_gemm_chunk_form(orc, pq, dev, N, K, T):
     y = pq.q8_gemm(w, qx, dx).cpu().numpy()
     bad = np.argwhere(_bits(y) != _bits(orc.q8_gemm(W, S, qx_r, dx_r)))
     assert bad.shape[0] == 0, f"{bad.shape[0]} cells differ, first {bad[:5].tolist()}"
+
+
+# The row-parallel form (long N): rows that end inside a tile and leave waves of
+# the last group without one, ragged positions, one chunk, one segment of 8 and
+# a ninth chunk in a second.
+@pytest.mark.parametrize("N,K,T", [(15900, 512, 256), (15872, 2304, 250), (16100, 256, 225), (32700, 2048, 128)])
+def test_gemm_row_form(orc, pq, dev, N, K, T):
+    print(f"gemm rows N={N} K={K} T={T}", flush=True)
+    W, S, w = _weights(orc, pq, dev, N, K, SEED + 3 * N + K)
+    x = orc.gen_normal(SEED + 9 * T + K, T * K).reshape(T, K)
+    qx_r, dx_r = orc.q8_quant(x)
+    qx, dx = pq.q8_quant(torch.from_numpy(x).to(dev))
+    y = pq.q8_gemm(w, qx, dx).cpu().numpy()
+    bad = np.argwhere(_bits(y) != _bits(orc.q8_gemm(W, S, qx_r, dx_r)))
+    assert bad.shape[0] == 0, f"{bad.shape[0]} cells differ, first {bad[:5].tolist()}"
