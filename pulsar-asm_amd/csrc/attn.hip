@@ -125,7 +125,7 @@ __global__ __launch_bounds__(64) void attn_split_kernel(const uint16_t *__restri
 //
 // What bounds it: per split and 32 rows 2 HD MFMA steps (64 cycles and more)
 // and about 1400 vector instructions (head_dim 64), 900 of them e^x. 512
-// queries from 0, 32 q and 8 kv heads of 64: 60.4 -> 27.8 us (a wave per query
+// queries from 0, 32 q and 8 kv heads of 64: 60.4 -> 25.6 us (a wave per query
 // read each K and V once per query and formed every chain on the vector unit).
 typedef float v16f __attribute__((ext_vector_type(16)));
 

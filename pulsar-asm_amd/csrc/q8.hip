@@ -778,7 +778,7 @@ __global__ __launch_bounds__(64 * S, 2) void q8_gemm_chunk_kernel(const int8_t *
 // whole chunks (a last chunk of fewer blocks costs registers that spill).
 // Against the walking form, whose waves take 32 rows: half the LDS reads of dx and
 // of the activations per output (they and the fold's instructions bound both):
-// 16384 x 2048 at 256 positions 40.1 -> 32.3 us (532 TOP/s), 65536 139 -> 121.
+// 16384 x 2048 at 256 positions 40.1 -> 33.1 us (519 TOP/s), 65536 139 -> 114.
 constexpr int kRwRows = 8 * kTR;
 
 __global__ __launch_bounds__(512, 2) void q8_gemm_rows_kernel(const int8_t *__restrict__ pc,
