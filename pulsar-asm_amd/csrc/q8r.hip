@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
 #pragma unroll
         for (int i = 0; i < BPL; i++) {
           const int b = L + 32 * i;
-          // a block past the chunk has zero codes and scale: fmaf(0, 0, acc) = acc
+          // a block past the chunk dots zero codes with block 0's x and leaves acc as it is (q8r_leaf)
           const float *xb = xp + (size_t)(b < nbc ? b : 0) * kRXStride;
           float dot = 0.0f;
 #pragma unroll
@@ -242,7 +242,8 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
               dot = __builtin_fmaf((float)(int8_t)(w >> 24), x4.w, dot);
             }
           }
-          acc = __builtin_fmaf(B.s[i], dot, acc);
+          const float next = __builtin_fmaf(B.s[i], dot, acc);
+          acc = b < nbc ? next : acc;
         }
         acc = leaf_tree32(acc);
         if (L == 0) ysum[(tt + p) * kRRows + wr] += acc;

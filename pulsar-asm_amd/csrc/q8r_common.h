@@ -62,8 +62,8 @@ __device__ __forceinline__ float q8r_leaf(const RBlocks &B, const float *__restr
 #pragma unroll
   for (int i = 0; i < BPL; i++) {
     const int b = L + 32 * i;
-    // a block past the chunk has zero codes and scale: fmaf(0, 0, acc) = acc
-    // exactly (acc is never -0), so it is folded without a branch
+    // a block past the chunk dots zero codes with block 0's x, without a branch,
+    // and leaves acc as it is by a select: 0 * x is NaN where that x is infinite
     const float *xb = xs + (size_t)(b < nbc ? c * nbc + b : 0) * kRXStride;
     const uint32_t w[8] = {(uint32_t)B.c[2 * i].x, (uint32_t)B.c[2 * i].y, (uint32_t)B.c[2 * i].z,
                            (uint32_t)B.c[2 * i].w, (uint32_t)B.c[2 * i + 1].x, (uint32_t)B.c[2 * i + 1].y,
@@ -77,7 +77,8 @@ __device__ __forceinline__ float q8r_leaf(const RBlocks &B, const float *__restr
       dot = __builtin_fmaf((float)(int8_t)((w[q] >> 16) & 0xffu), x4.z, dot);
       dot = __builtin_fmaf((float)(int8_t)(w[q] >> 24), x4.w, dot);
     }
-    acc = __builtin_fmaf(B.s[i], dot, acc);
+    const float next = __builtin_fmaf(B.s[i], dot, acc);
+    acc = b < nbc ? next : acc;
   }
   return acc;
 }

@@ -240,3 +240,21 @@ def test_q8r_matrix_matches_few_positions(pq, dev, N, K, T):
     y = pq.q8r_gemv(W, S, x, out_dtype=pq.DT_F32)
     want = torch.cat([pq.q8r_gemv(W, S, x[t:t + 8], out_dtype=pq.DT_F32) for t in range(0, T, 8)])
     assert torch.equal(y.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("T", [1, 2, 5, 6, 8, 9, 33])
+@pytest.mark.parametrize("N,K", [(40, 32), (77, 2080), (40, 7680)])
+def test_q8r_infinite_x_ragged_leaves(orc, pq, dev, N, K, T):
+    """A leaf without a block at its last place (nor, at K = 32, any block) adds nothing, whatever x
+    holds: an infinity in block 0 reaches a row through its own code alone, at any T."""
+    print(f"q8r infinite x N={N} K={K} T={T}", flush=True)
+    W, S, xb = _case(orc, N, K, T, SEED + 5 * N + K)
+    xb[:, 7] = 0x7f80
+    xb[T // 2, 7] = 0xff80
+    want = orc.q8r_gemm(W, S, xb)
+    inf = W[:, 7] != 0
+    assert np.isinf(want[:, inf]).all() and inf.any()
+    y = _run(pq, dev, W, S, xb, pq.DT_F32).cpu().numpy()
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(y), nan)
+    assert np.array_equal(y.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
