@@ -272,6 +272,11 @@ int pq_attn_decode(const uint16_t *q, int q_stride, const uint16_t *kcache, cons
                    const uint16_t *gate, int gate_stride, uint16_t *out, int out_stride, int8_t *qx,
                    float *dx, int pos0, int nh, int nkv, int hd, int T, float scale, int win, void *ws,
                    size_t ws_bytes, void *stream);
+/* Which kernel forms the partials of such a call (host arithmetic, no launch):
+ * 0 one wave per query, 1 matrix tiles (with a 16-byte aligned ws; else 0),
+ * -1 for sizes that pq_attn_decode refuses. The results are the same bits. No
+ * counterpart in the reference. */
+int pq_attn_decode_form(int nh, int nkv, int hd, int pos0, int T, int win);
 
 /* The reference-numerics arm's attention, in k_attn_head's own order
  * (lfm3_nanode.cu:503-602), then k_sigmoid_gate (852-858): pq_qk_prep_ref is

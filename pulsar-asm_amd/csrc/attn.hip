@@ -403,13 +403,29 @@ extern "C" size_t pq_attn_workspace_bytes(int nh, int hd, int max_pos, int T) {
 // from 1500 263 / 129; 16 and 4 heads of 128, 203 from 0 (1712) 23.1 / 25.2, 203 in
 // a window of 256 (4060) 33.2 / 34.2, 64 from 1500 (6400) 50.6 / 29.8, 512 from
 // 1500 235 / 128; 8 and 1 of 128, 203 from 0 (428) 22.1 / 23.3, 512 (2304) 39.3 / 29.6.
+// One query has as many tile waves as per-query ones. The per-query wave, which
+// costs by its heads, is then the cheaper one but for 8 heads, or 4 of 128 once
+// 4096 of its waves fill the chip: from 30000 keys 32 and 8 heads of 64 71.8 /
+// 72.8, from 64000 128 / 142, 32 and 32 from 16000 56.5 / 74.7, 32 and 16 of 128 from
+// 24000 85.0 / 115; 64 and 8 of 64 from 12500 45.2 / 37.0, 64 and 8 of 128 from 48000
+// 207 / 159, 16 and 4 of 128 from 66000 (4128 waves) 165 / 176, from 90000 272 / 228, 32
+// and 8 from 36000 (4504) 146 / 126. Two queries share the tiles: 32 and 8 of 64 from
+// 64000 161 / 143, 32 and 32 from 16000 85.5 / 77.3.
 static bool attn_tiles(int HD, int G, int nkv, int pos0, int T, int win) {
   auto splits = [&](long long npos) {
     const long long lo = win > 0 && npos > win ? npos - win : 0;
     return (npos + kSplit - 1) / kSplit - lo / kSplit;
   };
   const long long waves = nkv * (long long)T * (splits(pos0 + 1LL) + splits((long long)pos0 + T)) / 2;
+  if (T < 2 && G <= 4 && !(G == 4 && HD == 128 && waves >= 4500)) return false;
   return waves * (G > 4 ? 2 : 1) >= (HD == 64 ? 3072 : 4096);
+}
+
+extern "C" int pq_attn_decode_form(int nh, int nkv, int hd, int pos0, int T, int win) {
+  if (nkv <= 0 || nh <= 0 || nh % nkv || (hd != 64 && hd != 128) || pos0 < 0 || T <= 0 || win < 0) return -1;
+  const int G = nh / nkv;
+  if (G != 1 && G != 2 && G != 4 && G != 8) return -1;
+  return attn_tiles(hd, G, nkv, pos0, T, win) ? 1 : 0;
 }
 
 template <int HD>

@@ -62,6 +62,7 @@ SIGNATURES = {
     "pq_rmsnorm": (I, [P, P, P, P, P, P, P, I, I, F, P]),
     "pq_qk_prep": (I, [P, I, P, P, P, P, P, I, I, I, I, I, I, F, P]),
     "pq_attn_workspace_bytes": (Z, [I, I, I, I]),
+    "pq_attn_decode_form": (I, [I, I, I, I, I, I]),
     "pq_attn_decode": (I, [P, I, P, P, P, I, P, I, P, P, I, I, I, I, I, F, I, P, Z, P]),
     "pq_qk_prep_ref": (I, [P, I, P, P, P, P, P, I, I, I, I, I, I, F, P]),
     "pq_attn_ref": (I, [P, I, P, P, P, I, P, I, I, I, I, I, I, F, I, P]),

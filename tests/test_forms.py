@@ -1,0 +1,28 @@
+"""The rules that choose a kernel form, read through the library's form queries
+(host arithmetic: they run without a GPU)."""
+import pytest
+
+from pulsar_amd import lib
+
+
+@pytest.mark.parametrize("nh,nkv,hd,per_query,tiles", [
+    (32, 8, 64, 64000, None), (8, 8, 64, 64000, None), (32, 32, 64, 64000, None), (32, 16, 128, 64000, None),
+    (16, 4, 128, 66000, 90000), (32, 8, 128, 33000, 36000), (64, 8, 64, 12000, 12500), (64, 8, 128, 16000, 16500)])
+def test_attention_one_query(nh, nkv, hd, per_query, tiles):
+    """One query gives a matrix tile no second one to share its keys with: it takes tiles only
+    where they measured faster (8 heads a kv head, or 4 of 128 over many keys)."""
+    form = lib().pq_attn_decode_form
+    for pos0 in (0, 255, 1500, per_query):
+        assert form(nh, nkv, hd, pos0, 1, 0) == 0
+    if tiles is not None:
+        assert form(nh, nkv, hd, tiles, 1, 0) == 1
+    assert form(nh, nkv, hd, 64000, 64, 0) == 1
+    assert form(nh, nkv, hd, 0, 2, 0) == 0
+
+
+def test_attention_form_refuses_what_the_call_refuses():
+    form = lib().pq_attn_decode_form
+    for bad in ((24, 8, 64, 0, 4, 0), (32, 8, 96, 0, 4, 0), (30, 8, 64, 0, 4, 0), (32, 0, 64, 0, 4, 0),
+                (32, 8, 64, -1, 4, 0), (32, 8, 64, 0, 0, 0),
+                (32, 8, 64, 0, 4, -1)):
+        assert form(*bad) == -1

@@ -127,6 +127,8 @@ def test_attention(orc, pq, dev, npos_last, T, nh, nkv, hd, win):
     (8, 1, 128, 5, 700, 0, 0, False), (8, 1, 128, 900, 450, 256, 0, False), (32, 8, 64, 0, 400, 1, 0, True)])
 def test_attention_many_queries(pq, dev, nh, nkv, hd, pos0, T, win, pad, bad):
     print(f"attn tiles {nh}/{nkv}x{hd} pos0={pos0} T={T} win={win}", flush=True)
+    assert pq.lib().pq_attn_decode_form(nh, nkv, hd, pos0, T, win) == 1
+    assert pq.lib().pq_attn_decode_form(nh, nkv, hd, pos0 + T - 1, 1, win) == 0
     g = torch.Generator(device=dev)
     g.manual_seed(T + pos0 + hd)
     n, kvd, qs = pos0 + T, nkv * hd, nh * hd + pad
