@@ -59,6 +59,14 @@ int pq_check_bf16_cvt(uint32_t *counts, uint32_t *first, void *stream);
  * values, +-amax among them); counts/first per 256-block group as above
  * (first = the lowest mismatching thread). No counterpart in the reference. */
 int pq_check_quant_div(uint32_t *counts, uint32_t *first, uint32_t seed, void *stream);
+/* Self-check of the kernels' e^x (branch-free, v_ldexp_f32) against the steps
+ * of its definition over all 2^32 float bit patterns; counts/first per 65536
+ * patterns as in pq_check_bf16_cvt. sample: a device array of 65536 floats,
+ * sample[b] = the kernels' e^x of the pattern (b << 16) | (h(b) & 0xffff), h the
+ * integer hash x ^= x >> 16, x *= 0x7feb352d, x ^= x >> 15, x *= 0x846ca68b,
+ * x ^= x >> 16. Expected: no mismatch, NaN bits included. No counterpart in the
+ * reference. */
+int pq_check_expf(uint32_t *counts, uint32_t *first, float *sample, void *stream);
 /* The shader clock in MHz, measured by one wave over ~0.2 ms (cycle counter
  * against the 100 MHz real-time counter). out: 2 floats of device memory,
  * out[0] = MHz. No counterpart in the reference. */

@@ -96,12 +96,15 @@ __device__ __forceinline__ uint16_t f2h(float f) {
 // n = rint(x*log2 e), r = (x - n*ln2_hi) - n*ln2_lo, degree-7 Taylor
 // polynomial in Horner form, then the power of two, whose multiply alone
 // rounds (a subnormal result, once). Identical values on the host side, which
-// scales by two exact factors and branches; here v_ldexp_f32 and selects, so
-// that independent calls interleave (2^32 inputs compared: the same bits, NaN
-// for NaN; 1.55x the rate of the branches).
+// scales by two exact factors and branches; here v_ldexp_f32 and no branch, so
+// that independent calls interleave (1.66x the rate of the branches). x is
+// brought into [-105, 89], whose ends scale to 0 and infinity, so that the
+// integer conversion is of a small number whatever x is; a NaN is returned as
+// it is. pq_check_expf compares all 2^32 inputs.
 __device__ __forceinline__ float expf_pq(float x) {
-  const float n = __builtin_rintf(x * 1.44269502162933349609375f);
-  float r = __builtin_fmaf(n, -0.693145751953125f, x);
+  const float xc = __builtin_amdgcn_fmed3f(x, -105.0f, 89.0f);
+  const float n = __builtin_rintf(xc * 1.44269502162933349609375f);
+  float r = __builtin_fmaf(n, -0.693145751953125f, xc);
   r = __builtin_fmaf(n, -1.428606765330187045e-06f, r);
   float p = 1.98412698412698412e-4f;
   p = __builtin_fmaf(p, r, 1.38888888888888889e-3f);
@@ -111,9 +114,8 @@ __device__ __forceinline__ float expf_pq(float x) {
   p = __builtin_fmaf(p, r, 0.5f);
   p = __builtin_fmaf(p, r, 1.0f);
   p = __builtin_fmaf(p, r, 1.0f);
-  float y = __builtin_amdgcn_ldexpf(p, (int)n);
-  y = x > 88.72283935546875f ? __builtin_inff() : y;
-  return x < -104.0f ? 0.0f : y;
+  const float y = __builtin_amdgcn_ldexpf(p, (int)n);
+  return x != x ? x : y;
 }
 
 // Wave64 xor-butterfly reductions. After step k every aligned group of 2^k

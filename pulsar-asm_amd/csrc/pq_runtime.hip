@@ -126,6 +126,57 @@ __global__ __launch_bounds__(256) void quant_div_check_kernel(uint32_t *__restri
   }
 }
 
+// e^x by its definition's steps, as the host side writes them.
+__device__ float expf_steps(float x) {
+  if (x != x) return x;
+  if (x > 88.72283935546875f) return __builtin_inff();
+  if (x < -104.0f) return 0.0f;
+  const float n = __builtin_rintf(x * 1.44269502162933349609375f);
+  float r = __builtin_fmaf(n, -0.693145751953125f, x);
+  r = __builtin_fmaf(n, -1.428606765330187045e-06f, r);
+  float p = 1.98412698412698412e-4f;
+  p = __builtin_fmaf(p, r, 1.38888888888888889e-3f);
+  p = __builtin_fmaf(p, r, 8.33333333333333333e-3f);
+  p = __builtin_fmaf(p, r, 4.16666666666666667e-2f);
+  p = __builtin_fmaf(p, r, 1.66666666666666667e-1f);
+  p = __builtin_fmaf(p, r, 0.5f);
+  p = __builtin_fmaf(p, r, 1.0f);
+  p = __builtin_fmaf(p, r, 1.0f);
+  const int ni = (int)n, a = ni / 2, b = ni - a;
+  return (p * __uint_as_float((uint32_t)(a + 127) << 23)) * __uint_as_float((uint32_t)(b + 127) << 23);
+}
+
+// Block b: patterns b * 65536 and on, 256 per thread; sample[b] is expf_pq of
+// pattern b * 65536 + mix32(b) mod 65536.
+__global__ __launch_bounds__(256) void expf_check_kernel(uint32_t *__restrict__ counts, uint32_t *__restrict__ first,
+                                                         float *__restrict__ sample) {
+  __shared__ uint32_t sc[256], sf[256];
+  uint32_t n = 0, f = 0xffffffffu;
+  const uint32_t pick = mix32(blockIdx.x) & 0xffffu;
+  for (uint32_t i = 0; i < 256; i++) {
+    const uint32_t low = i * 256u + threadIdx.x, u = (blockIdx.x << 16) | low;
+    const float x = __uint_as_float(u), a = expf_pq(x), b = expf_steps(x);
+    const bool bad = __float_as_uint(a) != __float_as_uint(b);
+    n += bad ? 1u : 0u;
+    if (bad && u < f) f = u;
+    if (low == pick) sample[blockIdx.x] = a;
+  }
+  sc[threadIdx.x] = n;
+  sf[threadIdx.x] = f;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o) {
+      sc[threadIdx.x] += sc[threadIdx.x + o];
+      sf[threadIdx.x] = sf[threadIdx.x] < sf[threadIdx.x + o] ? sf[threadIdx.x] : sf[threadIdx.x + o];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    counts[blockIdx.x] = sc[0];
+    first[blockIdx.x] = sf[0];
+  }
+}
+
 // One wave: shader clock cycles (s_memtime) against the 100 MHz real-time
 // counter (s_memrealtime) over a bounded dependent-FMA loop of ~0.2 ms.
 __global__ __launch_bounds__(64) void clock_probe_kernel(float *__restrict__ out, int iters) {
@@ -182,6 +233,12 @@ extern "C" int pq_check_bf16_cvt(uint32_t *counts, uint32_t *first, void *stream
   PQ_REQUIRE(counts && first, PQ_ERR_ARG, "pq_check_bf16_cvt: null pointer");
   pq::launch(pq::bf16_cvt_check_kernel, dim3(65536), dim3(256), 0, pq::as_stream(stream), counts, first);
   return pq::check_launch("pq_check_bf16_cvt");
+}
+
+extern "C" int pq_check_expf(uint32_t *counts, uint32_t *first, float *sample, void *stream) {
+  PQ_REQUIRE(counts && first && sample, PQ_ERR_ARG, "pq_check_expf: null pointer");
+  pq::launch(pq::expf_check_kernel, dim3(65536), dim3(256), 0, pq::as_stream(stream), counts, first, sample);
+  return pq::check_launch("pq_check_expf");
 }
 
 extern "C" const char *pq_version(void) { return "pulsar-amd 0.1 gfx950"; }

@@ -52,6 +52,31 @@ def test_quant_shared_divisor_matches_division(pq, dev, seed):
     assert int(c.sum()) == 0, f"{int(c.sum())} mismatches; first threads {[int(x) for x in f[c > 0][:8]]}"
 
 
+def test_expf_exhaustive(orc, pq, dev):
+    """The kernels' e^x (x brought into range, v_ldexp_f32) equals the steps of its definition on all
+    2^32 inputs, infinities and NaN among them, and the oracle's on one input of every 65536."""
+    counts = torch.full((65536,), -1, dtype=torch.int32, device=dev)
+    first = torch.zeros(65536, dtype=torch.int32, device=dev)
+    sample = torch.zeros(65536, dtype=torch.float32, device=dev)
+    pq.check(pq.lib().pq_check_expf(counts.data_ptr(), first.data_ptr(), sample.data_ptr(), pq.stream_ptr()),
+             "pq_check_expf")
+    torch.cuda.synchronize()
+    c = counts.cpu().numpy().view(np.uint32)
+    f = first.cpu().numpy().view(np.uint32)
+    assert int(c.sum()) == 0, f"{int(c.sum())} mismatches, first {[hex(int(x)) for x in f[c > 0][:8]]}"
+    b = np.arange(65536, dtype=np.uint32)
+    h = b ^ (b >> 16)
+    h = h * np.uint32(0x7feb352d)
+    h = h ^ (h >> 15)
+    h = h * np.uint32(0x846ca68b)
+    h = h ^ (h >> 16)
+    x = ((b << 16) | (h & 0xffff)).view(np.float32)
+    got, want = sample.cpu().numpy(), orc.expf(x)
+    nan = np.isnan(x)
+    assert np.isnan(got[nan]).all() and np.isnan(want[nan]).all()
+    assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+
+
 def test_clock_probe(pq, dev):
     """pq_clock_mhz reports a shader clock in MI355X's range (its boost clock is 2.4 GHz)."""
     out = torch.zeros(2, dtype=torch.float32, device=dev)
