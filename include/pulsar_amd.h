@@ -168,6 +168,10 @@ int pq_q8_gemm_noalloc(const int8_t *pcodes, const uint16_t *pscales, const int8
  * (q8_partial_TLb, 4051-4509) on the shapes that use it. */
 int pq_q8r_gemv(const int8_t *codes, const float *scales, const uint16_t *x, void *y, int y_dtype, int N,
                 int K, int T, void *stream);
+/* Which kernels run such a call (host arithmetic, no launch): 0 the vector
+ * ones, 16 or 32 the matrix tile; -1 for sizes that pq_q8r_gemv refuses. The
+ * results are the same bits. No counterpart in the reference. */
+int pq_q8r_gemv_form(int N, int K, int T);
 
 /* ====================================================== Q4 / Q5 low-bit GEMV
  * The reference's low-bit backbone format and order (lfm3_qlow.cuh:1-113,

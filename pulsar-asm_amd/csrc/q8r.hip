@@ -265,6 +265,26 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
 
 using namespace pq;
 
+static int q8r_bpl(int K) { return (q8r_chunk(K) / kQ + 31) / 32; }   // blocks a leaf holds at most
+
+// Which form runs T positions: 0 the vector kernels, else the matrix tile. The
+// matrix cores pad T to 16 or 32 positions; below that the vector kernel costs
+// by the position. Per launch, vector / matrix: 2048 x 2048 at 8 positions 8.3 /
+// 9.0 us, 16384 x 2048 22.5 / 22.3, at 12 positions 512 x 2048 10.6 / 8.6; with
+// over 2 blocks a leaf (codes widened per use, 4.4 us a position at 2048 x 7680)
+// at 4 positions 17.4 / 24.3, at 8 30.9 / 24.7.
+static int q8r_form(int N, int K, int T) {
+  static const int env_t = env_int("PQ_Q8R_POSWISE");   // 1: one position per workgroup row at any T
+  return env_t != 1 && T > (q8r_bpl(K) <= 2 ? 8 : 5) ? q8r_mfma_tile(N, T) : 0;
+}
+
+extern "C" int pq_q8r_gemv_form(int N, int K, int T) {
+  if (N <= 0 || T <= 0 || K < kQ || K % kQ || q8r_bpl(K) > 8 || (long long)N * K >= (1ll << 31) ||
+      (size_t)(K / kQ) * kRXStride * sizeof(float) > kMaxLds)
+    return -1;
+  return q8r_form(N, K, T);
+}
+
 extern "C" int pq_q8r_gemv(const int8_t *codes, const float *scales, const uint16_t *x, void *y, int y_dtype, int N,
                            int K, int T, void *stream) {
   PQ_REQUIRE(codes && scales && x && y, PQ_ERR_ARG, "pq_q8r_gemv: null pointer");
@@ -273,21 +293,16 @@ extern "C" int pq_q8r_gemv(const int8_t *codes, const float *scales, const uint1
   PQ_REQUIRE(y_dtype == PQ_DTYPE_F32 || y_dtype == PQ_DTYPE_BF16, PQ_ERR_ARG, "pq_q8r_gemv: y_dtype %d", y_dtype);
   PQ_REQUIRE(aligned(codes, 16) && aligned(scales, 4) && aligned(x, 16) && K % 8 == 0, PQ_ERR_ALIGN,
              "pq_q8r_gemv: codes and x must be 16-byte aligned");
-  const int KC = q8r_chunk(K), bpl = (KC / kQ + 31) / 32;
+  const int KC = q8r_chunk(K), bpl = q8r_bpl(K);
   PQ_REQUIRE(bpl <= 8, PQ_ERR_ARG, "pq_q8r_gemv: K=%d (above 8192, K must be a multiple of 2048)", K);
   PQ_REQUIRE((long long)N * K < (1ll << 31), PQ_ERR_ARG, "pq_q8r_gemv: N=%d K=%d too large", N, K);
   const size_t lds = (size_t)(K / kQ) * kRXStride * sizeof(float);
   PQ_REQUIRE(lds <= kMaxLds, PQ_ERR_ARG, "pq_q8r_gemv: K=%d too large for LDS", K);
   const int yb = y_dtype == PQ_DTYPE_BF16 ? 1 : 0;
   hipStream_t st = as_stream(stream);
-  static const int env_t = env_int("PQ_Q8R_POSWISE");   // 1: one position per workgroup row at any T
-  if (T > 1 && env_t != 1) {   // each weight load serves many positions
-    // The matrix cores pad T to 16 or 32 positions; below that the vector
-    // kernel costs by the position. Per launch, vector / matrix: 2048 x 2048 at
-    // 8 positions 8.3 / 9.0 us, 16384 x 2048 22.5 / 22.3, at 12 positions 512 x
-    // 2048 10.6 / 8.6; with over 2 blocks a leaf (codes widened per use, 4.4 us
-    // a position at 2048 x 7680) at 4 positions 17.4 / 24.3, at 8 30.9 / 24.7.
-    if (T > (bpl <= 2 ? 8 : 5)) return q8r_mfma(codes, scales, x, y, yb, N, K, T, st);
+  if (const int mt = q8r_form(N, K, T)) return q8r_mfma(mt, codes, scales, x, y, yb, N, K, T, st);
+  static const int env_t = env_int("PQ_Q8R_POSWISE");
+  if (T > 1 && env_t != 1) {   // each weight load serves all positions
     // positions per LDS tile: as many 36-float padded chunks as fit 18 KB, at most 8 (small tiles keep
     // several workgroups per CU: 18 KB measured faster than 72 KB)
     const size_t per = (size_t)(KC / kQ) * kRXStride * sizeof(float);

@@ -17,8 +17,10 @@ constexpr int kRMaxChunks = 8;   // 2048-wide chunks a row may hold in the chunk
 
 __host__ __device__ inline int q8r_chunk(int K) { return (K >= 2048 && K % 2048 == 0) ? 2048 : K; }
 
-// The many-position form on the fp32 matrix cores (q8r_gemm.hip); yb: bf16 y.
-int q8r_mfma(const int8_t *codes, const float *scales, const uint16_t *x, void *y, int yb, int N, int K, int T,
+// The many-position form on the fp32 matrix cores (q8r_gemm.hip) in tiles of mt
+// = 16 or 32 rows x positions, and the tile to take; yb: bf16 y.
+int q8r_mfma_tile(int N, int T);
+int q8r_mfma(int mt, const int8_t *codes, const float *scales, const uint16_t *x, void *y, int yb, int N, int K, int T,
              hipStream_t st);
 
 struct RBlocks {

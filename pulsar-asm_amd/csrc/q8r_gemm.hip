@@ -316,12 +316,16 @@ static int q8r_mfma_go(const int8_t *codes, const float *scales, const uint16_t 
 // the busiest CU is taken. Measured, 32 / 16: 15360 x 2048 at 256 positions
 // 171 / 257 us, 4096 x 4096 at 48 28.4 / 28.5, 2048 x 8192 at 64 53 / 40,
 // 16384 x 2048 at 16 27 / 23, 2048 x 8192 at 32 53 / 29.
-int q8r_mfma(const int8_t *codes, const float *scales, const uint16_t *x, void *y, int yb, int N, int K, int T,
-             hipStream_t st) {
+int q8r_mfma_tile(int N, int T) {
   auto rounds = [&](int mt) {
     return ((long long)((N + mt - 1) / mt) * ((T + mt - 1) / mt) + 255) / 256;   // tiles of the busiest of 256 CUs
   };
-  if (2 * rounds(16) < 5 * rounds(32)) return q8r_mfma_go<16>(codes, scales, x, y, yb, N, K, T, st);
+  return 2 * rounds(16) < 5 * rounds(32) ? 16 : 32;
+}
+
+int q8r_mfma(int mt, const int8_t *codes, const float *scales, const uint16_t *x, void *y, int yb, int N, int K, int T,
+             hipStream_t st) {
+  if (mt == 16) return q8r_mfma_go<16>(codes, scales, x, y, yb, N, K, T, st);
   return q8r_mfma_go<32>(codes, scales, x, y, yb, N, K, T, st);
 }
 

@@ -53,6 +53,7 @@ SIGNATURES = {
     "pq_q8_gemm_workspace_bytes": (Z, [I, I, I]),
     "pq_q8_gemm_ws": (I, [P, P, P, P, P, I, I, I, I, P, Z, P]),
     "pq_q8r_gemv": (I, [P, P, P, P, I, I, I, I, P]),
+    "pq_q8r_gemv_form": (I, [I, I, I]),
     "pq_qlow_packed_codes_bytes": (Z, [I, I, I]),
     "pq_qlow_packed_scales_bytes": (Z, [I, I, I]),
     "pq_qlow_pack": (I, [P, P, I, I, I, P, P, P]),

@@ -26,10 +26,11 @@ def _run(pq, dev, W, S, xb, dt):
     return y
 
 
-# T > 1 runs the T-wide form (up to 32 positions per workgroup, x staged up to
-# 8 positions at a time): T = 40 and 33 cross both boundaries, K = 8192 and
-# 12288 fold several 2048-wide chunks, K = 7680 and 2560 are one chunk of 240
-# and 80 blocks (leaves with several blocks, codes widened per use); at T = 1
+# T = 2 .. 8 (5 with over 2 blocks a leaf) run the T-wide vector form, x staged
+# up to 8 positions at a time: one 2048-wide chunk of 8 positions fills several
+# stagings; more positions run the matrix form. K = 8192 and 12288 fold several
+# 2048-wide chunks, K = 7680 and 2560 are one chunk of 240 and 80 blocks (leaves
+# with several blocks, codes widened per use); at T = 1
 # rows of 2..8 chunks on few workgroups split their chunks over half-waves
 # (K = 4096, 6144: two per row; 8192, 12288, 16384: four); K = 5120, 7680
 # and 8160 are one chunk of 5..8 blocks per lane
@@ -37,10 +38,13 @@ def _run(pq, dev, W, S, xb, dt):
                                    (61, 512, 1), (37, 1024, 3), (13, 32, 1), (65, 12288, 1), (45, 2560, 2),
                                    (2048, 2048, 4), (300, 2048, 40), (77, 8192, 33), (97, 7680, 9),
                                    (64, 12288, 5), (45, 2560, 17), (300, 4096, 1), (33, 16384, 1),
-                                   (7, 6144, 1), (2048, 7680, 1), (131, 5120, 1), (40, 8160, 1)])
+                                   (7, 6144, 1), (2048, 7680, 1), (131, 5120, 1), (40, 8160, 1),
+                                   (65, 2048, 8), (300, 1024, 8), (33, 6144, 8), (97, 7680, 5), (15, 8160, 4),
+                                   (9, 2080, 5), (12, 96, 8)])
 def test_q8r_gemv_bitexact(orc, pq, dev, N, K, T):
     print(f"q8r N={N} K={K} T={T}", flush=True)
     W, S, xb = _case(orc, N, K, T, SEED + N + K, signed_scales=(N % 2 == 1))
+    assert (pq.lib().pq_q8r_gemv_form(N, K, T) == 0) == (T <= (8 if K <= 2048 or K % 2048 == 0 else 5))
     want = orc.q8r_gemm(W, S, xb)
     y = _run(pq, dev, W, S, xb, pq.DT_F32).cpu().numpy()
     assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
@@ -197,23 +201,28 @@ def test_q8r_gemv_fused_embed(pq, dev, K):
         assert torch.equal(y.view(torch.int16), want.view(torch.int16)), tok
 
 
-# The matrix-core form (more than 8 positions; 5 with over 2 blocks a leaf):
-# 16- and 32-wide tiles at their edges (one row or position more or less than
-# a tile), ragged leaves (65 and 9 blocks a chunk, one block, a class without
-# blocks), several chunks.
-@pytest.mark.parametrize("N,K,T", [(1, 32, 9), (15, 288, 16), (17, 2080, 17), (31, 2048, 33), (33, 4096, 31),
-                                   (64, 7680, 6), (16, 8160, 12), (40, 8192, 9), (2100, 256, 65), (520, 6144, 129)])
-def test_q8r_matrix_tiles(orc, pq, dev, N, K, T):
-    print(f"q8r matrix N={N} K={K} T={T}", flush=True)
+# The matrix-core form (more than 8 positions; 5 with over 2 blocks a leaf), by
+# the tile that the call takes: 16- and 32-wide ones at their edges (one row or
+# position more or less than a tile), ragged leaves (65, 9, 240 and 255 blocks a
+# chunk, one block, a class without blocks), several chunks.
+@pytest.mark.parametrize("tile,N,K,T", [
+    (16, 1, 32, 9), (16, 15, 288, 16), (16, 17, 2080, 17), (16, 31, 2048, 33), (16, 33, 4096, 31), (16, 64, 7680, 6),
+    (16, 16, 8160, 12), (16, 40, 8192, 9), (16, 520, 6144, 129), (32, 2100, 256, 65), (32, 2049, 288, 65),
+    (32, 2100, 2080, 65), (32, 2079, 2048, 96), (32, 2100, 6144, 65), (32, 2081, 7680, 66), (32, 2051, 8160, 65)])
+def test_q8r_matrix_tiles(orc, pq, dev, tile, N, K, T):
+    print(f"q8r matrix tile={tile} N={N} K={K} T={T}", flush=True)
+    assert pq.lib().pq_q8r_gemv_form(N, K, T) == tile
     W, S, xb = _case(orc, N, K, T, SEED + 3 * N + K, signed_scales=True)
     want = orc.q8r_gemm(W, S, xb)
     y = _run(pq, dev, W, S, xb, pq.DT_F32).cpu().numpy()
     assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
 
 
-def test_q8r_matrix_exponents(orc, pq, dev):
+@pytest.mark.parametrize("tile,N,K,T", [(16, 70, 2048, 40), (32, 2060, 2048, 68), (32, 2060, 2336, 68)])
+def test_q8r_matrix_exponents(orc, pq, dev, tile, N, K, T):
     """x over the whole exponent range: sums that round at every step, subnormal products and sums, overflow."""
-    N, K, T = 70, 2048, 40
+    print(f"q8r exponents tile={tile} N={N} K={K} T={T}", flush=True)
+    assert pq.lib().pq_q8r_gemv_form(N, K, T) == tile
     W, S, xb = _case(orc, N, K, T, SEED + 77, signed_scales=True)
     e = orc.gen_codes(SEED + 78, T * K).reshape(T, K).astype(np.int32)
     e[: T // 4] //= 8                       # +-15: every step rounds
@@ -229,16 +238,22 @@ def test_q8r_matrix_exponents(orc, pq, dev):
     assert np.array_equal(y.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
 
 
-@pytest.mark.parametrize("N,K,T", [(16416, 512, 96), (8200, 1024, 40)])
-def test_q8r_matrix_matches_few_positions(pq, dev, N, K, T):
-    """More tiles than workgroups: the same bits as the vector kernel's, 8 positions at a time."""
+@pytest.mark.parametrize("tile,N,K,T", [(32, 16416, 512, 96), (16, 8200, 1024, 40), (32, 8200, 4096, 65),
+                                        (32, 8200, 2080, 67), (16, 8200, 4096, 40)])
+def test_q8r_matrix_matches_few_positions(pq, dev, tile, N, K, T):
+    """More tiles than workgroups (512 of 32-wide ones, 1024 of 16-wide), so a workgroup goes on to another tile
+    from its last chunk: the same bits as the vector kernel's, 5 positions at a time."""
+    print(f"q8r tiles walk tile={tile} N={N} K={K} T={T}", flush=True)
+    L = pq.lib()
+    assert L.pq_q8r_gemv_form(N, K, T) == tile and L.pq_q8r_gemv_form(N, K, 5) == 0
+    assert (N + 8 * tile - 1) // (8 * tile) * 8 * ((T + tile - 1) // tile) > {32: 512, 16: 1024}[tile]
     g = torch.Generator(device=dev)
     g.manual_seed(N + K)
     W = torch.randint(-127, 128, (N, K), dtype=torch.int8, device=dev, generator=g)
     S = torch.rand((N, K // 32), device=dev, generator=g) * 0.02
     x = torch.randn((T, K), device=dev, generator=g).to(torch.bfloat16)
     y = pq.q8r_gemv(W, S, x, out_dtype=pq.DT_F32)
-    want = torch.cat([pq.q8r_gemv(W, S, x[t:t + 8], out_dtype=pq.DT_F32) for t in range(0, T, 8)])
+    want = torch.cat([pq.q8r_gemv(W, S, x[t:t + 5], out_dtype=pq.DT_F32) for t in range(0, T, 5)])
     assert torch.equal(y.view(torch.int32), want.view(torch.int32))
 
 
