@@ -134,6 +134,11 @@ int pq_q8_gemm(const int8_t *pcodes, const uint16_t *pscales, const int8_t *qx, 
  * counterpart of the reference's chunked partials + k_combine_bf_T
  * (lfm3_nanode.cu:4840-4968). */
 size_t pq_q8_gemm_workspace_bytes(int N, int K, int T);
+/* Which kernel runs such a call (host arithmetic, no launch): 1 the walking
+ * one, 2 + 16 * waves the chunk-parallel one and the waves of its tile (4 or
+ * 8), 3 the one of 32-row slices, 4 the row-parallel one; -1 for sizes that are
+ * refused. The results are the same bits. No counterpart in the reference. */
+int pq_q8_gemm_form(int N, int K, int T);
 int pq_q8_gemm_ws(const int8_t *pcodes, const uint16_t *pscales, const int8_t *qx, const float *dx,
                   void *y, int y_dtype, int N, int K, int T, void *ws, size_t ws_bytes, void *stream);
 
@@ -207,6 +212,10 @@ int pq_qlow_gemv_ws(const uint8_t *pcodes, const uint16_t *pscales, const uint16
  * of pf_gemv_T for a low-bit source tensor (lfm3_nanode.cu:4846-4848). */
 int pq_qlow_gemm(const uint8_t *pcodes, const uint16_t *pscales, const uint16_t *x, void *y, int y_dtype, int N,
                  int K, int T, int ldy, int bits, void *stream);
+/* Which kernel runs such a call (host arithmetic, no launch): 0 the vector one,
+ * 16 or 32 the matrix tile; -1 for a shape that is refused. The results are the
+ * same bits. No counterpart in the reference. */
+int pq_qlow_gemm_form(int N, int K, int T, int bits);
 
 /* ============================================================ weight blob
  * The .lfm3q8 file the reference's exporter writes (export_lfm3_q8.py) and

@@ -1028,6 +1028,18 @@ static int gemm_form(int N, int K, int T) {
   return t_rw < t_wk ? kFormRows : kFormWalk;
 }
 
+// Waves of a chunk-parallel tile: 8 (one workgroup per CU) while the tiles fit
+// the CUs once, else 4 (two per CU). Measured, 4 / 8 waves: 2048 x 8192 at 256
+// positions (256 tiles) 29.2 / 20.8 us, at 512 (512) 39.9 / 42.2; 6144 x 2048 at
+// 64 (192) 8.8 / 6.9, at 96 (288) 11.6 / 12.5.
+static int chunk_waves(int N, int T) { return (long long)ntiles(N) * ((T + 31) / 32) <= 256 ? 8 : 4; }
+
+extern "C" int pq_q8_gemm_form(int N, int K, int T) {
+  if (N <= 0 || K <= 0 || K % kQ || T <= 0) return -1;
+  const int form = gemm_form(N, K, T);
+  return form == kFormChunk ? form + 16 * chunk_waves(N, T) : form;
+}
+
 extern "C" size_t pq_q8_gemm_workspace_bytes(int N, int K, int T) {
   if (N <= 0 || K <= 0 || K % kQ || T <= 0) return 0;
   if (gemm_form(N, K, T) != kFormWalk) return 0;
@@ -1061,12 +1073,9 @@ extern "C" int pq_q8_gemm_ws(const int8_t *pcodes, const uint16_t *pscales, cons
     return check_launch("pq_q8_gemm");
   }
   if (form == kFormChunk) {
-    // 8 waves a tile (one workgroup per CU) while the tiles fit the CUs once, else 4 (two per CU). Measured, 4 / 8
-    // waves: 2048 x 8192 at 256 positions (256 tiles) 29.2 / 20.8 us, at 512 (512) 39.9 / 42.2; 6144 x 2048 at 64 (192)
-    // 8.8 / 6.9, at 96 (288) 11.6 / 12.5
     const int npt = (T + 31) / 32;
     const dim3 grid((unsigned)((ntiles(N) + 7) / 8 * 8 * npt));
-    if ((long long)ntiles(N) * npt <= 256)
+    if (chunk_waves(N, T) == 8)
       launch(q8_gemm_chunk_kernel<8>, grid, dim3(512), 8 * kCkWave, st, pcodes, pscales, qx, dx, y, yb, N, K, T, npt);
     else
       launch(q8_gemm_chunk_kernel<4>, grid, dim3(256), 4 * kCkWave, st, pcodes, pscales, qx, dx, y, yb, N, K, T, npt);

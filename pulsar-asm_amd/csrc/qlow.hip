@@ -905,6 +905,19 @@ static void qlow_gemm_shape(int N, int K, int T, int &RS, int &TB) {
   }
 }
 
+// The matrix tile that a call takes (qlow_mfma_tile), or 0 and the vector
+// kernel's (RS, TB).
+static int qlow_gemm_tile(int N, int K, int T, int &RS, int &TB) {
+  qlow_gemm_shape(N, K, T, RS, TB);
+  const long long rv = ((long long)(N / RS) * ((T + TB - 1) / TB) + 255) / 256;
+  return qlow_mfma_tile(N, K, T, qlow_ks(K), rv, RS, TB);
+}
+
+extern "C" int pq_qlow_gemm_form(int N, int K, int T, int bits) {
+  int RS, TB;
+  return qlow_shape(N, K, bits) && T > 0 ? qlow_gemm_tile(N, K, T, RS, TB) : -1;
+}
+
 extern "C" int pq_qlow_gemm(const uint8_t *pcodes, const uint16_t *pscales, const uint16_t *x, void *y,
                             int y_dtype, int N, int K, int T, int ldy, int bits, void *stream) {
   PQ_REQUIRE(pcodes && pscales && x && y, PQ_ERR_ARG, "pq_qlow_gemm: null pointer");
@@ -917,9 +930,7 @@ extern "C" int pq_qlow_gemm(const uint8_t *pcodes, const uint16_t *pscales, cons
   PQ_REQUIRE(aligned(pcodes, 16) && aligned(pscales, 4) && aligned(x, 16), PQ_ERR_ALIGN,
              "pq_qlow_gemm: packed codes and x must be 16-byte aligned");
   int RS, TB;
-  qlow_gemm_shape(N, K, T, RS, TB);
-  const long long rv = ((long long)(N / RS) * ((T + TB - 1) / TB) + 255) / 256;
-  if (const int mt = qlow_mfma_tile(N, K, T, qlow_ks(K), rv, RS, TB))
+  if (const int mt = qlow_gemm_tile(N, K, T, RS, TB))
     return qlow_mfma(mt, pcodes, reinterpret_cast<const uint32_t *>(pscales), x, y, y_dtype == PQ_DTYPE_BF16 ? 1 : 0,
                      N, K, T, ldy, bits, qlow_ks(K), as_stream(stream));
   const int G = K / kQ, XL = (K / 8 + kQgNT - 1) / kQgNT;

@@ -51,6 +51,7 @@ SIGNATURES = {
     "pq_q8_gemv": (I, [P, P, P, P, P, I, I, I, P]),
     "pq_q8_gemm": (I, [P, P, P, P, P, I, I, I, I, P]),
     "pq_q8_gemm_workspace_bytes": (Z, [I, I, I]),
+    "pq_q8_gemm_form": (I, [I, I, I]),
     "pq_q8_gemm_ws": (I, [P, P, P, P, P, I, I, I, I, P, Z, P]),
     "pq_q8r_gemv": (I, [P, P, P, P, I, I, I, I, P]),
     "pq_q8r_gemv_form": (I, [I, I, I]),
@@ -61,6 +62,7 @@ SIGNATURES = {
     "pq_qlow_workspace_bytes": (Z, [I, I, I]),
     "pq_qlow_gemv_ws": (I, [P, P, P, P, I, I, I, I, P, Z, P]),
     "pq_qlow_gemm": (I, [P, P, P, P, I, I, I, I, I, I, P]),
+    "pq_qlow_gemm_form": (I, [I, I, I, I]),
     "pq_rmsnorm": (I, [P, P, P, P, P, P, P, I, I, F, P]),
     "pq_qk_prep": (I, [P, I, P, P, P, P, P, I, I, I, I, I, I, F, P]),
     "pq_attn_workspace_bytes": (Z, [I, I, I, I]),

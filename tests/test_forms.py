@@ -26,3 +26,23 @@ def test_attention_form_refuses_what_the_call_refuses():
                 (32, 8, 64, -1, 4, 0), (32, 8, 64, 0, 0, 0),
                 (32, 8, 64, 0, 4, -1)):
         assert form(*bad) == -1
+
+
+def test_gemm_forms_refuse_what_the_calls_refuse():
+    L = lib()
+    for bad in ((0, 2048, 4), (64, 2040, 4), (64, 2048, 0)):
+        assert L.pq_q8_gemm_form(*bad) == -1 and L.pq_q8r_gemv_form(*bad) == -1
+        assert L.pq_qlow_gemm_form(*bad, 4) == -1
+    assert L.pq_q8r_gemv_form(8, 8992, 4) == -1                 # over 8 blocks a leaf
+    assert L.pq_qlow_gemm_form(64, 2048, 4, 6) == -1 and L.pq_qlow_gemm_form(64, 16640, 4, 4) == -1
+
+
+def test_gemm_workspace_only_for_the_walking_form():
+    """No other form of the Q8_0 GEMM splits K over workgroups through memory."""
+    L = lib()
+    for N in (1, 300, 3104, 8000, 16384, 40000):
+        for K in (32, 2048, 8192):
+            for T in (1, 32, 33, 97, 256):
+                if L.pq_q8_gemm_form(N, K, T) != 1:
+                    assert L.pq_q8_gemm_workspace_bytes(N, K, T) == 0
+    assert L.pq_q8_gemm_form(2048, 8192, 32) == 1 and L.pq_q8_gemm_workspace_bytes(2048, 8192, 32) > 0

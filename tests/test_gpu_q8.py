@@ -119,7 +119,9 @@ def test_gemv_repeat_and_inplace(orc, pq, dev):
                                    # the LFM3 shapes: FFN 7680 (gate+up 15360 rows, down K = 7680),
                                    # q|k|v|gate 3088 rows, vocab 128000
                                    (15360, 2048, 32), (2048, 7680, 32), (2048, 7680, 256), (3088, 2048, 100),
-                                   (128000, 2048, 32)])
+                                   (128000, 2048, 32),
+                                   # the walking form over several position blocks, a last chunk of one block
+                                   (16320, 288, 97)])
 def test_gemm_bitexact(orc, pq, dev, N, K, T):
     print(f"gemm N={N} K={K} T={T}", flush=True)
     W, S, w = _weights(orc, pq, dev, N, K, SEED + 11 * N + K)
@@ -143,10 +145,13 @@ def test_gemm_bitexact(orc, pq, dev, N, K, T):
 # The chunk-parallel form (more than 32 positions) at its edges: 4 and 8 waves a
 # tile, one row and one position past a tile, fewer chunks than waves, a last
 # chunk of 1, 7 and 8 blocks, several rounds of chunks.
-@pytest.mark.parametrize("N,K,T", [(1, 32, 33), (65, 224, 64), (64, 256, 65), (127, 2080, 100), (300, 4384, 40),
-                                   (16320, 288, 97), (2112, 2304, 300), (4160, 8192, 129), (520, 16384, 36)])
-def test_gemm_chunk_form(orc, pq, dev, N, K, T):
-    print(f"gemm chunks N={N} K={K} T={T}", flush=True)
+@pytest.mark.parametrize("waves,N,K,T", [
+    (8, 1, 32, 33), (8, 65, 224, 64), (8, 64, 256, 65), (8, 127, 2080, 100), (8, 300, 4384, 40), (8, 520, 16384, 36),
+    (4, 8000, 32, 97), (4, 8000, 288, 97), (4, 4097, 1024, 161), (4, 2112, 2304, 300), (4, 8031, 2272, 97),
+    (4, 4160, 8192, 129)])
+def test_gemm_chunk_form(orc, pq, dev, waves, N, K, T):
+    print(f"gemm chunks waves={waves} N={N} K={K} T={T}", flush=True)
+    assert pq.lib().pq_q8_gemm_form(N, K, T) == 2 + 16 * waves
     W, S, w = _weights(orc, pq, dev, N, K, SEED + 7 * N + K)
     x = orc.gen_normal(SEED + 5 * T + K, T * K).reshape(T, K)
     qx_r, dx_r = orc.q8_quant(x)
@@ -162,6 +167,7 @@ def test_gemm_chunk_form(orc, pq, dev, N, K, T):
 @pytest.mark.parametrize("N,K,T", [(15900, 512, 256), (15872, 2304, 250), (16100, 256, 225), (32700, 2048, 128)])
 def test_gemm_row_form(orc, pq, dev, N, K, T):
     print(f"gemm rows N={N} K={K} T={T}", flush=True)
+    assert pq.lib().pq_q8_gemm_form(N, K, T) == 4
     W, S, w = _weights(orc, pq, dev, N, K, SEED + 3 * N + K)
     x = orc.gen_normal(SEED + 9 * T + K, T * K).reshape(T, K)
     qx_r, dx_r = orc.q8_quant(x)

@@ -220,10 +220,13 @@ def test_qlow_gemm_equals_gemv(orc, pq, dev, bits, N, K, T):
 # 34 groups, not a multiple of the 4 taken at once; an odd number of row tiles)
 # and 32-wide ones (2 and 4 slices, ragged positions), at both widths of code.
 # K = 16384 is the longest row.
-@pytest.mark.parametrize("bits,N,K,T", [(5, 2048, 4352, 33), (4, 2080, 2048, 65), (5, 4128, 512, 49), (4, 1024, 16384, 65),
-                                        (4, 16384, 256, 64), (5, 16416, 256, 97), (5, 4096, 4352, 255), (4, 4096, 4096, 256)])
-def test_qlow_matrix_tiles(pq, dev, bits, N, K, T):
-    print(f"qlow matrix bits={bits} N={N} K={K} T={T}", flush=True)
+@pytest.mark.parametrize("tile,bits,N,K,T", [
+    (16, 5, 2048, 4352, 33), (16, 4, 2080, 2048, 65), (16, 5, 4128, 512, 49), (16, 4, 1024, 16384, 65),
+    (32, 4, 16384, 256, 64), (32, 5, 16416, 256, 97), (32, 5, 4096, 4352, 255), (32, 4, 4096, 4096, 256)])
+def test_qlow_matrix_tiles(pq, dev, tile, bits, N, K, T):
+    print(f"qlow matrix tile={tile} bits={bits} N={N} K={K} T={T}", flush=True)
+    assert pq.lib().pq_qlow_gemm_form(N, K, T, bits) == tile
+    assert pq.lib().pq_qlow_gemm_form(N, K, 2, bits) == (16 if K == 256 else 0)
     g = torch.Generator(device=dev)
     g.manual_seed(N + K + T + bits)
     Q = torch.randint(0, 1 << bits, (N, K), dtype=torch.uint8, device=dev, generator=g)
@@ -239,21 +242,23 @@ def test_qlow_matrix_tiles(pq, dev, bits, N, K, T):
         assert torch.equal(wide[t, :N].view(torch.int32), pq.qlow_gemv(w, X[t], out_dtype=pq.DT_F32).view(torch.int32)), t
         assert torch.equal(yb[t].view(torch.int16), pq.qlow_gemv(w, X[t]).view(torch.int16)), t
     assert torch.isnan(wide[:, N:]).all()
-    first = pq.qlow_gemm(w, X[:2], out_dtype=pq.DT_F32)   # the vector form
+    first = pq.qlow_gemm(w, X[:2], out_dtype=pq.DT_F32)   # the vector form, but at K = 256
     assert torch.equal(first.view(torch.int32), wide[:2, :N].contiguous().view(torch.int32))
 
 
-def test_qlow_matrix_infinity(pq, dev):
+@pytest.mark.parametrize("tile,N,T", [(16, 4096, 40), (32, 16384, 70)])
+def test_qlow_matrix_infinity(pq, dev, tile, N, T):
     """An infinite or NaN x reaches its own position's outputs only."""
+    assert pq.lib().pq_qlow_gemm_form(N, 2048, T, 4) == tile
     g = torch.Generator(device=dev)
     g.manual_seed(5)
-    w = pq.QlowWeight(torch.randint(0, 16, (4096, 2048), dtype=torch.uint8, device=dev, generator=g),
-                      (torch.randn((4096, 64, 2), device=dev, generator=g) * 0.05).half(), 4)
-    X = torch.randn((40, 2048), device=dev, generator=g).to(torch.bfloat16)
+    w = pq.QlowWeight(torch.randint(0, 16, (N, 2048), dtype=torch.uint8, device=dev, generator=g),
+                      (torch.randn((N, 64, 2), device=dev, generator=g) * 0.05).half(), 4)
+    X = torch.randn((T, 2048), device=dev, generator=g).to(torch.bfloat16)
     want = pq.qlow_gemm(w, X, out_dtype=pq.DT_F32)
     X[7, 100], X[33, 2047] = float("inf"), float("nan")
     y = pq.qlow_gemm(w, X, out_dtype=pq.DT_F32)
-    keep = [t for t in range(40) if t not in (7, 33)]
+    keep = [t for t in range(T) if t not in (7, 33)]
     assert torch.equal(y[keep].view(torch.int32), want[keep].view(torch.int32))
     for t in (7, 33):
         one = pq.qlow_gemv(w, X[t], out_dtype=pq.DT_F32)
