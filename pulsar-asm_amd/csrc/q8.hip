@@ -485,9 +485,9 @@ __global__ __launch_bounds__(kGemmThreads) void q8_gemm_kernel(const int8_t *__r
     }
 }
 
-// The tile-parallel form (one position block): a workgroup = S 32-row
-// slices x 32 positions, 8*S waves; wave w takes slice w % S and chunk
-// 8*rd + w / S of round rd, so a round's 8 chunks of every slice load at once.
+// The tile-parallel form (one position block): a workgroup = one 32-row slice
+// x 32 positions, 8 waves; wave w takes chunk 8*rd + w of round rd, so a
+// round's 8 chunks load at once.
 // Per round the 32 positions' activations (2048 K) and dx are loaded first,
 // then the wave's weights, so the staging waits only on the activations; the
 // 8 chunk partials then fold into y through LDS in chunk order (the partials
@@ -500,36 +500,33 @@ constexpr int kTileSlots = 8;
 constexpr size_t kTileActBytes = 32 * (size_t)kGemmARow;
 constexpr size_t kTileLds = kTileActBytes + (size_t)kTileSlots * kCB * 32 * 4;
 
-template <int S, bool PIPE, int PH = 32>
-__global__ __launch_bounds__(64 * kTileSlots * S) void q8_gemm_tile_kernel(const int8_t *__restrict__ pc,
+template <bool PIPE, int PH = 32>
+__global__ __launch_bounds__(64 * kTileSlots) void q8_gemm_tile_kernel(const int8_t *__restrict__ pc,
                                                                         const uint16_t *__restrict__ ps,
                                                                         const int8_t *__restrict__ qx,
                                                                         const float *__restrict__ dx,
                                                                         void *__restrict__ y, int y_bf16, int N,
                                                                         int K, int T) {
-  constexpr int NT = 64 * kTileSlots * S;
+  constexpr int NT = 64 * kTileSlots;
   constexpr int APT = 32 * (kGemmSegK / 16) / NT;   // 16-byte activation pieces per thread per round
   constexpr int DPT = 32 * kTileSlots * kCB / NT;   // dx entries per thread per round
-  static_assert(kTileSlots * S * 16 * 64 * 4 <= kTileActBytes, "partials must fit the activation buffer");
+  static_assert(kTileSlots * 16 * 64 * 4 <= kTileActBytes, "partials must fit the activation buffer");
   extern __shared__ __align__(16) unsigned char gsm[];
   int8_t(*as)[kGemmARow] = reinterpret_cast<int8_t(*)[kGemmARow]>(gsm);
-  float(*part)[S][16][64] = reinterpret_cast<float(*)[S][16][64]>(gsm);   // aliases as
+  float(*part)[16][64] = reinterpret_cast<float(*)[16][64]>(gsm);   // aliases as
   float(*dxs)[32] = reinterpret_cast<float(*)[32]>(gsm + kTileActBytes);
   const int nb = K / kQ, nch = nchunks(K);
   static_assert(PH == 32 || PH == 16, "16 or 32 positions per workgroup");
   constexpr int NQ = PH / 8;                          // position quads folded per lane
   const int p0 = blockIdx.z * PH;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int sub = wave % S, slot = wave / S;
+  const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int h = lane >> 5, l32 = lane & 31;
-  const int sl = blockIdx.x * S + sub;                 // 32-row slice
-  const bool live = sl * 32 < N;
-  const int tile = live ? sl >> 1 : 0, jt = (sl & 1) * 32 + l32;
+  const int sl = blockIdx.x, tile = sl >> 1, jt = (sl & 1) * 32 + l32;   // the 32-row slice, half of a tile
   const int np = T - p0 < PH ? T - p0 : PH;   // rows past np of the A operand read zeros
   const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<int8_t *>(pc + (size_t)tile * nb * kSlab), (short)0, live ? nb * kSlab : 0, kRsrcWord3);
+      const_cast<int8_t *>(pc + (size_t)tile * nb * kSlab), (short)0, nb * kSlab, kRsrcWord3);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t *>(ps + (size_t)tile * nch * kTR * 8), (short)0, live ? nch * kTR * 16 : 0, kRsrcWord3);
+      const_cast<uint16_t *>(ps + (size_t)tile * nch * kTR * 8), (short)0, nch * kTR * 16, kRsrcWord3);
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int8_t *>(qx + (size_t)p0 * K), (short)0, np * K, kRsrcWord3);
   const __amdgpu_buffer_rsrc_t rdx = __builtin_amdgcn_make_buffer_rsrc(
@@ -583,23 +580,23 @@ __global__ __launch_bounds__(64 * kTileSlots * S) void q8_gemm_tile_kernel(const
     }
     lds_barrier();   // every wave is done with the activations: the partials overwrite them
 #pragma unroll
-    for (int r = 0; r < 16; r++) part[slot][sub][r][lane] = a[r];
+    for (int r = 0; r < 16; r++) part[slot][r][lane] = a[r];
     lds_barrier();
     const int n = nch - rbase < kTileSlots ? nch - rbase : kTileSlots;
 #pragma unroll
     for (int k = 0; k < 2; k++) {
       const int e = t + k * NT;
-      const int s2 = e >> 10, r = (e >> 6) & 15, l = e & 63;
+      const int r = e >> 6, l = e & 63;
       if ((r >> 2) < NQ)
-        for (int w = 0; w < n; w++) yv[k] = yv[k] + part[w][s2][r][l];
+        for (int w = 0; w < n; w++) yv[k] = yv[k] + part[w][r][l];
     }
   }
 #pragma unroll
   for (int k = 0; k < 2; k++) {
     const int e = t + k * NT;
-    const int s2 = e >> 10, r = (e >> 6) & 15, l = e & 63;
+    const int r = e >> 6, l = e & 63;
     const int pos = p0 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
-    const int row = (blockIdx.x * S + s2) * 32 + (l & 31);
+    const int row = sl * 32 + (l & 31);
     if ((r >> 2) < NQ && pos < T && row < N) {
       if (y_bf16) reinterpret_cast<uint16_t *>(y)[(size_t)pos * N + row] = f2bf(yv[k]);
       else reinterpret_cast<float *>(y)[(size_t)pos * N + row] = yv[k];
@@ -1089,13 +1086,13 @@ extern "C" int pq_q8_gemm_ws(const int8_t *pcodes, const uint16_t *pscales, cons
     static const int env_ph = env_int("PQ_GEMM_PH");
     const long long items32 = (long long)((N + 31) / 32) * ((T + 31) / 32);
     if (env_ph != 32 && (env_ph == 16 ? items32 <= 256 : items32 <= 128))
-      launch(q8_gemm_tile_kernel<1, true, 16>, dim3((unsigned)((N + 31) / 32), 1, (unsigned)((T + 15) / 16)),
+      launch(q8_gemm_tile_kernel<true, 16>, dim3((unsigned)((N + 31) / 32), 1, (unsigned)((T + 15) / 16)),
              dim3(64 * kTileSlots), kTileLds, st, pcodes, pscales, qx, dx, y, yb, N, K, T);
     else if (items32 <= 256)
-      launch(q8_gemm_tile_kernel<1, true>, dim3((unsigned)((N + 31) / 32), 1, (unsigned)((T + 31) / 32)),
+      launch(q8_gemm_tile_kernel<true>, dim3((unsigned)((N + 31) / 32), 1, (unsigned)((T + 31) / 32)),
              dim3(64 * kTileSlots), kTileLds, st, pcodes, pscales, qx, dx, y, yb, N, K, T);
     else
-      launch(q8_gemm_tile_kernel<1, false>, dim3((unsigned)((N + 31) / 32), 1, (unsigned)((T + 31) / 32)),
+      launch(q8_gemm_tile_kernel<false>, dim3((unsigned)((N + 31) / 32), 1, (unsigned)((T + 31) / 32)),
              dim3(64 * kTileSlots), kTileLds, st, pcodes, pscales, qx, dx, y, yb, N, K, T);
     return check_launch("pq_q8_gemm");
   }
