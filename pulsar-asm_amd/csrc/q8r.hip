@@ -154,14 +154,19 @@ __global__ __launch_bounds__(kRThreads * CW) void q8r_gemv_kc_kernel(const int8_
 
 // The T-wide form for a few positions (more run on the matrix cores,
 // q8r_gemm.hip): the same per-output arithmetic, with each weight load serving
-// all positions. A workgroup takes 8 rows x up to kRTPW positions; per chunk
+// all positions. A workgroup takes 8 rows x the T <= kRTPW positions; per chunk
 // of K its lanes load their leaves' blocks once (CVT: codes widened to fp32
 // once, for up to 2 blocks per leaf), then the positions' x of that chunk are
 // staged in LDS tp at a time (bf16 widened to fp32, 36-float padded blocks) and
 // every position runs the leaf chains and the tree of the single-position
 // kernel. The chunk partials of a (position, row) go to an LDS running sum in
 // chunk order, y = ((0 + p_0) + p_1) + ...
-constexpr int kRTPW = 8;       // positions per workgroup
+constexpr int kRTPW = 8;       // positions at most
+
+// Blocks of LDS that a staged position takes: those of a chunk, and where some
+// leaf lacks one a block of zeros that it reads instead (another block's x may be
+// infinite, and 0 * x a NaN; q8r_leaf's select here costs 1% at 2 .. 8 positions).
+__host__ __device__ inline int q8r_pos_blocks(int nbc, int bpl) { return nbc < 32 * bpl ? nbc + 1 : nbc; }
 
 template <int BPL, bool CVT>
 __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__restrict__ codes,
@@ -171,15 +176,18 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
   extern __shared__ __align__(16) float rsm[];
   const int nb = K / kQ, KC = q8r_chunk(K), nbc = KC / kQ, nch = K / KC;
   float *ysum = rsm;                                   // [kRTPW][kRRows] running sums
-  float *xs = rsm + kRTPW * kRRows;                    // [tp][nbc][kRXStride]
+  const int nbs = q8r_pos_blocks(nbc, BPL);
+  float *xs = rsm + kRTPW * kRRows;                    // [tp][nbs][kRXStride]
   const int wr = threadIdx.x >> 5, L = threadIdx.x & 31;
   const int row = blockIdx.x * kRRows + wr;
-  const int t0 = blockIdx.y * kRTPW, tn = T - t0 < kRTPW ? T - t0 : kRTPW;
   const __amdgpu_buffer_rsrc_t rc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(codes), (short)0, N * K, kRsrcWord3);
   const __amdgpu_buffer_rsrc_t rs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(scales), (short)0, N * nb * 4, kRsrcWord3);
   for (int i = threadIdx.x; i < kRTPW * kRRows; i += kRThreads) ysum[i] = 0.0f;
+  if (nbs > nbc)
+    for (int i = threadIdx.x; i < tp * 32; i += kRThreads)
+      xs[((size_t)(i >> 5) * nbs + nbc) * kRXStride + (i & 31)] = 0.0f;
   for (int c = 0; c < nch; c++) {
     RBlocks B;
     q8r_load<BPL>(B, rc, rs, row, N, K, nb, nbc, c, L);
@@ -194,13 +202,13 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
         for (int k = 0; k < 32; k++) cf[i][k] = (float)(int8_t)((w[k >> 2] >> (8 * (k & 3))) & 0xffu);
       }
     }
-    for (int tt = 0; tt < tn; tt += tp) {
-      const int np = tn - tt < tp ? tn - tt : tp;
+    for (int tt = 0; tt < T; tt += tp) {
+      const int np = T - tt < tp ? T - tt : tp;
       __syncthreads();   // the previous tile's reads of xs are done (and ysum is zeroed)
-      // x of positions t0+tt .. +np, chunk c: 8 bf16 per thread per step
+      // x of positions tt .. +np, chunk c: 8 bf16 per thread per step
       for (int e = threadIdx.x * 8; e < np * KC; e += kRThreads * 8) {
         const int p = e / KC, k = e % KC;
-        const uint4 u = *reinterpret_cast<const uint4 *>(x + (size_t)(t0 + tt + p) * K + (size_t)c * KC + k);
+        const uint4 u = *reinterpret_cast<const uint4 *>(x + (size_t)(tt + p) * K + (size_t)c * KC + k);
         const uint32_t v[4] = {u.x, u.y, u.z, u.w};
         float f[8];
 #pragma unroll
@@ -208,19 +216,20 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
           f[2 * q] = __uint_as_float(v[q] << 16);
           f[2 * q + 1] = __uint_as_float(v[q] & 0xffff0000u);
         }
-        float *d = xs + ((size_t)p * nbc + (k >> 5)) * kRXStride + (k & 31);
+        float *d = xs + ((size_t)p * nbs + (k >> 5)) * kRXStride + (k & 31);
         *reinterpret_cast<float4 *>(d) = make_float4(f[0], f[1], f[2], f[3]);
         *reinterpret_cast<float4 *>(d + 4) = make_float4(f[4], f[5], f[6], f[7]);
       }
       __syncthreads();
       for (int p = 0; p < np; p++) {
-        const float *xp = xs + (size_t)p * nbc * kRXStride;
+        const float *xp = xs + (size_t)p * nbs * kRXStride;
         float acc = 0.0f;
 #pragma unroll
         for (int i = 0; i < BPL; i++) {
           const int b = L + 32 * i;
-          // a block past the chunk dots zero codes with block 0's x and leaves acc as it is (q8r_leaf)
-          const float *xb = xp + (size_t)(b < nbc ? b : 0) * kRXStride;
+          // a block past the chunk has zero codes, scale and x: fmaf(0, 0, acc) = acc but for the sign of a zero, which
+          // the sum of the chunks from 0 drops
+          const float *xb = xp + (size_t)(b < nbc ? b : nbc) * kRXStride;
           float dot = 0.0f;
 #pragma unroll
           for (int q = 0; q < 8; q++) {
@@ -242,8 +251,7 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
               dot = __builtin_fmaf((float)(int8_t)(w >> 24), x4.w, dot);
             }
           }
-          const float next = __builtin_fmaf(B.s[i], dot, acc);
-          acc = b < nbc ? next : acc;
+          acc = __builtin_fmaf(B.s[i], dot, acc);
         }
         acc = leaf_tree32(acc);
         if (L == 0) ysum[(tt + p) * kRRows + wr] += acc;
@@ -251,12 +259,12 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < tn * kRRows; i += kRThreads) {
+  for (int i = threadIdx.x; i < T * kRRows; i += kRThreads) {
     const int t = i / kRRows, r = blockIdx.x * kRRows + i % kRRows;
     if (r < N) {
       const float v = ysum[i];
-      if (y_bf16) reinterpret_cast<uint16_t *>(y)[(size_t)(t0 + t) * N + r] = f2bf(v);
-      else reinterpret_cast<float *>(y)[(size_t)(t0 + t) * N + r] = v;
+      if (y_bf16) reinterpret_cast<uint16_t *>(y)[(size_t)t * N + r] = f2bf(v);
+      else reinterpret_cast<float *>(y)[(size_t)t * N + r] = v;
     }
   }
 }
@@ -275,7 +283,7 @@ static int q8r_bpl(int K) { return (q8r_chunk(K) / kQ + 31) / 32; }   // blocks 
 // at 4 positions 17.4 / 24.3, at 8 30.9 / 24.7.
 static int q8r_form(int N, int K, int T) {
   static const int env_t = env_int("PQ_Q8R_POSWISE");   // 1: one position per workgroup row at any T
-  return env_t != 1 && T > (q8r_bpl(K) <= 2 ? 8 : 5) ? q8r_mfma_tile(N, T) : 0;
+  return env_t != 1 && T > (q8r_bpl(K) <= 2 ? kRTPW : 5) ? q8r_mfma_tile(N, T) : 0;
 }
 
 extern "C" int pq_q8r_gemv_form(int N, int K, int T) {
@@ -305,16 +313,17 @@ extern "C" int pq_q8r_gemv(const int8_t *codes, const float *scales, const uint1
   if (T > 1 && env_t != 1) {   // each weight load serves all positions
     // positions per LDS tile: as many 36-float padded chunks as fit 18 KB, at most 8 (small tiles keep
     // several workgroups per CU: 18 KB measured faster than 72 KB)
-    const size_t per = (size_t)(KC / kQ) * kRXStride * sizeof(float);
+    const int lb = bpl <= 1 ? 1 : bpl <= 2 ? 2 : bpl <= 4 ? 4 : 8;   // the kernel's blocks a leaf
+    const size_t per = (size_t)q8r_pos_blocks(KC / kQ, lb) * kRXStride * sizeof(float);
     static const int env_kb = env_int("PQ_Q8R_TILE_KB");
     const size_t budget = (size_t)(env_kb > 0 ? env_kb : 18) * 1024;
     const int tp = (int)std::min<size_t>(8, std::max<size_t>(1, budget / per));
     const size_t lds_t = (size_t)kRTPW * kRRows * sizeof(float) + (size_t)tp * per;
     PQ_REQUIRE(lds_t <= kMaxLds, PQ_ERR_ARG, "pq_q8r_gemv: K=%d too large for LDS", K);
-    const dim3 gt((unsigned)((N + kRRows - 1) / kRRows), (unsigned)((T + kRTPW - 1) / kRTPW)), bt(kRThreads);
-    if (bpl <= 1) launch(q8r_gemm_kernel<1, true>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
-    else if (bpl <= 2) launch(q8r_gemm_kernel<2, true>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
-    else if (bpl <= 4) launch(q8r_gemm_kernel<4, false>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
+    const dim3 gt((unsigned)((N + kRRows - 1) / kRRows)), bt(kRThreads);
+    if (lb == 1) launch(q8r_gemm_kernel<1, true>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
+    else if (lb == 2) launch(q8r_gemm_kernel<2, true>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
+    else if (lb == 4) launch(q8r_gemm_kernel<4, false>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
     else launch(q8r_gemm_kernel<8, false>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
     return check_launch("pq_q8r_gemv");
   }
