@@ -304,11 +304,12 @@ int pq_attn_decode_form(int nh, int nkv, int hd, int pos0, int T, int win);
  * pq_qk_prep with the cache holding the bf16 k and v rows as k_kv_write copies
  * them (157-162); pq_attn_ref attends query t (row t of q) at position pos0+t
  * to keys lo..pos0+t of that bf16 cache (lo as in pq_attn_decode) with one
- * 1024-thread workgroup per (head, t): each score a chain over the lane's
- * hd/32 dims and the shfl_down tree of a 32-lane warp (32 warps share the
- * keys); then its first 256 threads keep the reference's places: the softmax
- * sum per thread over keys t, t+256, ..., the warp tree, the 8 warps' tree;
- * the probabilities normalized before an 8-segment value sum added pairwise. e^x is the build's expf_pq where the reference
+ * workgroup of 1024, 512 or 256 threads (fewer when there are many) per (head,
+ * t): each score a chain over the lane's hd/32 dims and the shfl_down tree of a
+ * 32-lane warp (all warps share the keys); then its first 256 threads keep the
+ * reference's places: the softmax sum per thread over keys t, t+256, ..., the
+ * warp tree, the 8 warps' tree; the probabilities normalized before an
+ * 8-segment value sum added pairwise. e^x is the build's expf_pq where the reference
  * calls CUDA's expf. head_dim 64 or 128; at most 32768 keys in a window;
  * gate NULL for none; out bf16 [T] rows of stride out_stride. */
 int pq_qk_prep_ref(uint16_t *qkv, int row_stride, const float *q_norm, const float *k_norm,

@@ -418,10 +418,14 @@ static int attn_ref_launch(const uint16_t *q, int q_stride, const uint16_t *kcac
   const AttnGate g = gq != nullptr ? *gq : AttnGate{};
   // Many workgroups: fewer threads each, so that a CU holds several and one's
   // score, softmax and value phases (8 waves at most work on the last) run beside
-  // another's. Measured at 1024 / 512 / 256 threads (with the value sums on 4 waves):
-  // 16 heads of 128, 203 queries in a window of 256 (3248 workgroups) 44.3 / 36.0 / 34.3 us, 512 from 0 (8192) 128 /
-  // 97 / 90; 32 heads of 64, 512 from 0 209 / 157 / 143; 8 heads of 64, 64 from 1500
-  // (512) 32.9 / 32.1 / 33.0; 16 heads of 128, 16 from 1500 (256) 23.9 / 24.9 / 32.1.
+  // another's. Measured at 1024 / 512 / 256 threads (us): 16 heads of 128, 16 queries
+  // from 1500 (256 workgroups) 16.8 / 16.8 / 25.0, 24 (384) 25.7 / 25.6 / 28.0, 32 (512)
+  // 26.1 / 26.3 / 28.8, 48 (768) 37.2 / 35.3 / 39.1, 64 (1024) 47.3 / 43.9 / 48.2, from 0
+  // 12.6 / 9.1 / 6.8, in a window of 256 14.8 / 12.3 / 12.0; 203 (3248) from 1500 145 /
+  // 130 / 130, from 0 36.6 / 27.2 / 19.5, in the window 40.0 / 31.5 / 26.7; 32 heads of 64,
+  // 32 queries (1024) from 1500 37.5 / 33.2 / 36.3, from 0 10.9 / 8.3 / 6.1, 512 from 0 196 /
+  // 133 / 95.7. So 512 threads cost nothing from 512 workgroups on; 256 lose up to a
+  // tenth over 1500 keys at 1024 workgroups and win a quarter over short contexts.
   const long long wgs = (long long)nh * T;
   const int nt = pp != nullptr || wgs < 512 ? kArThreads : wgs < 1024 ? 512 : 256;
 #define PQ_ARN(HH, TT)                                                                                  \

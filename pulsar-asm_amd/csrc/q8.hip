@@ -619,7 +619,9 @@ __global__ __launch_bounds__(64 * kTileSlots) void q8_gemm_tile_kernel(const int
 // issued: one register set, loads a chunk ahead. Against 64-row tiles of 16
 // waves that staged 2048 K for all and folded unpipelined: 2048 x 8192 at 256
 // positions 28.3 -> 20.8 us, 3104 x 2048 at 512 31.5 -> 21.0 (310 TOP/s), 2048 x
-// 2048 at 64 7.5 -> 6.7.
+// 2048 at 64 7.5 -> 6.7. The ragged last chunk's copy of the loop beside the whole
+// one's takes the kernel to 256 VGPRs and 8 (S = 8) or 12 (S = 4) of them to
+// scratch; with whole chunks alone it compiles to 220 and 224 and spills none.
 constexpr int kCkRow = kCB * kQ + 16;                          // padded LDS row of a position's chunk (bytes)
 constexpr int kCkWave = 32 * kCkRow + kCB * 32 * 4;            // a wave's LDS: activations, then dx [8][32]
 
@@ -775,7 +777,7 @@ __global__ __launch_bounds__(64 * S, 2) void q8_gemm_chunk_kernel(const int8_t *
 // whole chunks (a last chunk of fewer blocks costs registers that spill).
 // Against the walking form, whose waves take 32 rows: half the LDS reads of dx and
 // of the activations per output (they and the fold's instructions bound both):
-// 16384 x 2048 at 256 positions 40.1 -> 33.1 us (519 TOP/s), 65536 139 -> 114.
+// 16384 x 2048 at 256 positions 37.1 -> 32.0 us (537 TOP/s), 65536 134 -> 118.
 constexpr int kRwRows = 8 * kTR;
 
 __global__ __launch_bounds__(512, 2) void q8_gemm_rows_kernel(const int8_t *__restrict__ pc,
@@ -1008,10 +1010,11 @@ enum { kFormWalk = 1, kFormChunk = 2, kFormSlice = 3, kFormRows = 4 };
 // share of the chip, the row-parallel form's rounds of 256 workgroups (a round's
 // waves are bound by their own chains when few, by the CU when all run), the
 // walking form's rounds where it would not split K. Measured, walking / chunk /
-// row (us, * taken): 16384 x 2048 at 64 positions 26.2 / 13.6* / 25.7, at 96 43.3 /
-// 20.4* / 26.4, at 128 20.9* / 26.2 / 27.0, at 256 40.1 / 46.5 / 32.3*; 15360 at 256 -
-// / 39.3 / 31.2*; 65536 at 64 46.2 / 45.1 / 36.7*, at 256 139 / 153 / 121*; 6144 at 512
-// - / 31.4 / 30.6*; 3104 at 512 - / 20.4* / 27.3.
+// row (us, * taken): 16384 x 2048 at 64 positions 27.0 / 13.3* / 25.6, at 96 42.4 /
+// 19.0* / 26.2, at 128 20.6* / 25.0 / 26.9, at 256 37.1 / 42.5 / 32.0*; 15360 at 256
+// 43.6 / 38.7 / 30.9*; 65536 at 64 44.5 / 42.7 / 35.6*, at 256 134 / 146 / 118*; 6144 at
+// 512 32.2 / 31.2 / 30.0*; 3104 at 512 44.5 / 20.2* / 26.6. (2048 x 8192 at 33 to 64
+// positions, which the walking form would split: 14.0 to 15.3 / 18.2* / 85.)
 static int gemm_form(int N, int K, int T) {
   static const int env = env_int("PQ_GEMM_FORM");
   if ((env >= kFormWalk && env <= kFormSlice) || (env == kFormRows && K % (kCB * kQ) == 0)) return env;
