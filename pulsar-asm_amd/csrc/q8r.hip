@@ -163,12 +163,13 @@ __global__ __launch_bounds__(kRThreads * CW) void q8r_gemv_kc_kernel(const int8_
 // chunk order, y = ((0 + p_0) + p_1) + ...
 constexpr int kRTPW = 8;       // positions at most
 
-// Blocks of LDS that a staged position takes: those of a chunk, and where some
-// leaf lacks one a block of zeros that it reads instead (another block's x may be
-// infinite, and 0 * x a NaN; q8r_leaf's select here costs 1% at 2 .. 8 positions).
-__host__ __device__ inline int q8r_pos_blocks(int nbc, int bpl) { return nbc < 32 * bpl ? nbc + 1 : nbc; }
-
-template <int BPL, bool CVT>
+// RAG: some leaf has fewer than BPL blocks. Its missing ones dot zero codes with
+// block 0's x and are dropped by q8r_leaf's select, which costs 1% where it is
+// not needed (a staged block of zeros in its place cost more: 16384 x 512 at 8
+// positions 8.9 -> 10.2 us). Without RAG the offset keeps its select all the
+// same: with b alone the loop comes out slower (2048 x 8192 at 8 positions 27.1 ->
+// 33.0 us).
+template <int BPL, bool CVT, bool RAG>
 __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__restrict__ codes,
                                                              const float *__restrict__ scales,
                                                              const uint16_t *__restrict__ x, void *__restrict__ y,
@@ -176,8 +177,7 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
   extern __shared__ __align__(16) float rsm[];
   const int nb = K / kQ, KC = q8r_chunk(K), nbc = KC / kQ, nch = K / KC;
   float *ysum = rsm;                                   // [kRTPW][kRRows] running sums
-  const int nbs = q8r_pos_blocks(nbc, BPL);
-  float *xs = rsm + kRTPW * kRRows;                    // [tp][nbs][kRXStride]
+  float *xs = rsm + kRTPW * kRRows;                    // [tp][nbc][kRXStride]
   const int wr = threadIdx.x >> 5, L = threadIdx.x & 31;
   const int row = blockIdx.x * kRRows + wr;
   const __amdgpu_buffer_rsrc_t rc =
@@ -185,9 +185,6 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
   const __amdgpu_buffer_rsrc_t rs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(scales), (short)0, N * nb * 4, kRsrcWord3);
   for (int i = threadIdx.x; i < kRTPW * kRRows; i += kRThreads) ysum[i] = 0.0f;
-  if (nbs > nbc)
-    for (int i = threadIdx.x; i < tp * 32; i += kRThreads)
-      xs[((size_t)(i >> 5) * nbs + nbc) * kRXStride + (i & 31)] = 0.0f;
   for (int c = 0; c < nch; c++) {
     RBlocks B;
     q8r_load<BPL>(B, rc, rs, row, N, K, nb, nbc, c, L);
@@ -216,20 +213,18 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
           f[2 * q] = __uint_as_float(v[q] << 16);
           f[2 * q + 1] = __uint_as_float(v[q] & 0xffff0000u);
         }
-        float *d = xs + ((size_t)p * nbs + (k >> 5)) * kRXStride + (k & 31);
+        float *d = xs + ((size_t)p * nbc + (k >> 5)) * kRXStride + (k & 31);
         *reinterpret_cast<float4 *>(d) = make_float4(f[0], f[1], f[2], f[3]);
         *reinterpret_cast<float4 *>(d + 4) = make_float4(f[4], f[5], f[6], f[7]);
       }
       __syncthreads();
       for (int p = 0; p < np; p++) {
-        const float *xp = xs + (size_t)p * nbs * kRXStride;
+        const float *xp = xs + (size_t)p * nbc * kRXStride;
         float acc = 0.0f;
 #pragma unroll
         for (int i = 0; i < BPL; i++) {
           const int b = L + 32 * i;
-          // a block past the chunk has zero codes, scale and x: fmaf(0, 0, acc) = acc but for the sign of a zero, which
-          // the sum of the chunks from 0 drops
-          const float *xb = xp + (size_t)(b < nbc ? b : nbc) * kRXStride;
+          const float *xb = xp + (size_t)(b < nbc ? b : 0) * kRXStride;
           float dot = 0.0f;
 #pragma unroll
           for (int q = 0; q < 8; q++) {
@@ -251,7 +246,8 @@ __global__ __launch_bounds__(kRThreads) void q8r_gemm_kernel(const int8_t *__res
               dot = __builtin_fmaf((float)(int8_t)(w >> 24), x4.w, dot);
             }
           }
-          acc = __builtin_fmaf(B.s[i], dot, acc);
+          const float next = __builtin_fmaf(B.s[i], dot, acc);
+          acc = RAG && b >= nbc ? acc : next;
         }
         acc = leaf_tree32(acc);
         if (L == 0) ysum[(tt + p) * kRRows + wr] += acc;
@@ -313,18 +309,21 @@ extern "C" int pq_q8r_gemv(const int8_t *codes, const float *scales, const uint1
   if (T > 1 && env_t != 1) {   // each weight load serves all positions
     // positions per LDS tile: as many 36-float padded chunks as fit 18 KB, at most 8 (small tiles keep
     // several workgroups per CU: 18 KB measured faster than 72 KB)
-    const int lb = bpl <= 1 ? 1 : bpl <= 2 ? 2 : bpl <= 4 ? 4 : 8;   // the kernel's blocks a leaf
-    const size_t per = (size_t)q8r_pos_blocks(KC / kQ, lb) * kRXStride * sizeof(float);
+    const size_t per = (size_t)(KC / kQ) * kRXStride * sizeof(float);
     static const int env_kb = env_int("PQ_Q8R_TILE_KB");
     const size_t budget = (size_t)(env_kb > 0 ? env_kb : 18) * 1024;
     const int tp = (int)std::min<size_t>(8, std::max<size_t>(1, budget / per));
     const size_t lds_t = (size_t)kRTPW * kRRows * sizeof(float) + (size_t)tp * per;
     PQ_REQUIRE(lds_t <= kMaxLds, PQ_ERR_ARG, "pq_q8r_gemv: K=%d too large for LDS", K);
     const dim3 gt((unsigned)((N + kRRows - 1) / kRRows)), bt(kRThreads);
-    if (lb == 1) launch(q8r_gemm_kernel<1, true>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
-    else if (lb == 2) launch(q8r_gemm_kernel<2, true>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
-    else if (lb == 4) launch(q8r_gemm_kernel<4, false>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
-    else launch(q8r_gemm_kernel<8, false>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp);
+#define PQ_RG(BB, CC, RR) launch(q8r_gemm_kernel<BB, CC, RR>, gt, bt, lds_t, st, codes, scales, x, y, yb, N, K, T, tp)
+    if (KC / kQ == 32) PQ_RG(1, true, false);
+    else if (KC / kQ == 64) PQ_RG(2, true, false);
+    else if (bpl <= 1) PQ_RG(1, true, true);
+    else if (bpl <= 2) PQ_RG(2, true, true);
+    else if (bpl <= 4) PQ_RG(4, false, true);
+    else PQ_RG(8, false, true);   // no chunk of 128 or 256 blocks: K = 4096 and 8192 have chunks of 64
+#undef PQ_RG
     return check_launch("pq_q8r_gemv");
   }
   const dim3 grid((unsigned)((N + kRRows - 1) / kRRows), (unsigned)T), block(kRThreads);
