@@ -136,8 +136,9 @@ int pq_q8_gemm(const int8_t *pcodes, const uint16_t *pscales, const int8_t *qx, 
 size_t pq_q8_gemm_workspace_bytes(int N, int K, int T);
 /* Which kernel runs such a call (host arithmetic, no launch): 1 the walking
  * one, 2 + 16 * waves the chunk-parallel one and the waves of its tile (4 or
- * 8), 3 the one of 32-row slices, 4 the row-parallel one; -1 for sizes that are
- * refused. The results are the same bits. No counterpart in the reference. */
+ * 8), 3 the one of 32-row slices, 4 the row-parallel one (2 and 4: + 256 where
+ * their work is split evenly over the XCDs and not by whole row groups); -1 for
+ * sizes that are refused. The results are the same bits. No counterpart in the reference. */
 int pq_q8_gemm_form(int N, int K, int T);
 int pq_q8_gemm_ws(const int8_t *pcodes, const uint16_t *pscales, const int8_t *qx, const float *dx,
                   void *y, int y_dtype, int N, int K, int T, void *ws, size_t ws_bytes, void *stream);

@@ -662,20 +662,46 @@ __device__ __forceinline__ void chunk2(float (*a)[16], v4i (*w)[kCB], const v4i 
   }
 }
 
+// Workgroup b's row group and position block, of ng x npt (false: none). The
+// workgroups go round-robin over the 8 XCDs; a group's position blocks run on
+// one XCD, whose L2 serves the group's weights again: XCD x takes groups x,
+// x + 8, ..., or with `even` the x-th eighth of all items in group order (a
+// group then on two XCDs at most), so that none has more items than its share.
+__device__ __forceinline__ bool group_of(int b, int ng, int npt, int even, int &group, int &pos) {
+  const int total = ng * npt, k = b >> 3, i = even ? (b & 7) * ((total + 7) / 8) + k : k;
+  group = i / npt;
+  pos = i - group * npt;
+  if (!even) group = group * 8 + (b & 7);
+  return group < ng;
+}
+
+// The even split where it saves a round of workgroups (per_cu of them a CU) on
+// the XCD with the most groups. Measured, whole groups / even: 3104 x 2048 at 160
+// positions (35 of 245 workgroups for one XCD's 32 CUs) 12.6 / 7.6 us, at 320 16.1 /
+// 11.7, 2100 x 8192 at 224 35.4 / 19.4, 13000 x 2048 at 160 24.7 / 20.2, 8200 x 2048 at
+// 384 (row-parallel) 44.2 / 26.7; with as many rounds, 33000 x 2048 at 256 78.2 / 81.7.
+static int group_even(long long ng, long long npt, int per_cu) {
+  const long long slots = 32 * per_cu;
+  return (ng * npt + 8 * slots - 1) / (8 * slots) < ((ng + 7) / 8 * npt + slots - 1) / slots ? 1 : 0;
+}
+static unsigned group_grid(int ng, int npt, int even) {
+  return (unsigned)(even ? (ng * npt + 7) / 8 * 8 : (ng + 7) / 8 * 8 * npt);
+}
+
 template <int S>
 __global__ __launch_bounds__(64 * S, 2) void q8_gemm_chunk_kernel(const int8_t *__restrict__ pc,
                                                                    const uint16_t *__restrict__ ps,
                                                                    const int8_t *__restrict__ qx,
                                                                    const float *__restrict__ dx, void *__restrict__ y,
-                                                                   int y_bf16, int N, int K, int T, int npt) {
+                                                                   int y_bf16, int N, int K, int T, int npt,
+                                                                   int even) {
   constexpr int NQ4 = 512 / (64 * S);   // float4s of the 64 x 32 outputs per thread
   static_assert(kCkWave >= 2048 * 4, "a wave's partials reuse its LDS");
   extern __shared__ __align__(16) unsigned char gsm[];
   const int nb = K / kQ, nch = nchunks(K);
-  // workgroups go round-robin over the 8 XCDs: the position tiles of a row tile run on one XCD, whose L2 serves its
-  // weights again
-  const int idx = blockIdx.x >> 3, tile = (idx / npt) * 8 + (blockIdx.x & 7), t0 = (idx % npt) * 32;
-  if (tile * kTR >= N) return;
+  int tile, pb;
+  if (!group_of(blockIdx.x, (N + kTR - 1) / kTR, npt, even, tile, pb)) return;
+  const int t0 = pb * 32;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int h = lane >> 5, l32 = lane & 31;
   unsigned char *mine = gsm + wave * kCkWave;
@@ -784,14 +810,14 @@ __global__ __launch_bounds__(512, 2) void q8_gemm_rows_kernel(const int8_t *__re
                                                                const uint16_t *__restrict__ ps,
                                                                const int8_t *__restrict__ qx,
                                                                const float *__restrict__ dx, void *__restrict__ y,
-                                                               int y_bf16, int N, int K, int T, int npt) {
+                                                               int y_bf16, int N, int K, int T, int npt, int even) {
   extern __shared__ __align__(16) unsigned char gsm[];
   int8_t(*as)[kGemmARow] = reinterpret_cast<int8_t(*)[kGemmARow]>(gsm);              // [32 positions]
   float(*dxs)[32] = reinterpret_cast<float(*)[32]>(gsm + 32 * kGemmARow);            // [64 blocks][32]
   const int nb = K / kQ, nch = nchunks(K);
-  // the position blocks of a group of rows run on one XCD (workgroup id mod 8), whose L2 serves its weights again
-  const int idx = blockIdx.x >> 3, gr = (idx / npt) * 8 + (blockIdx.x & 7), t0 = (idx % npt) * 32;
-  if (gr * kRwRows >= N) return;
+  int gr, pb;
+  if (!group_of(blockIdx.x, (N + kRwRows - 1) / kRwRows, npt, even, gr, pb)) return;
+  const int t0 = pb * 32;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int h = lane >> 5, l32 = lane & 31;
   const bool live = gr * kRwRows + wave * kTR < N;   // a wave past N reads zeros and writes nothing
@@ -1036,8 +1062,9 @@ static int chunk_waves(int N, int T) { return (long long)ntiles(N) * ((T + 31) /
 
 extern "C" int pq_q8_gemm_form(int N, int K, int T) {
   if (N <= 0 || K <= 0 || K % kQ || T <= 0) return -1;
-  const int form = gemm_form(N, K, T);
-  return form == kFormChunk ? form + 16 * chunk_waves(N, T) : form;
+  const int form = gemm_form(N, K, T), npt = (T + 31) / 32, waves = chunk_waves(N, T);
+  if (form == kFormRows) return form + 256 * group_even((N + kRwRows - 1) / kRwRows, npt, 1);
+  return form == kFormChunk ? form + 16 * waves + 256 * group_even(ntiles(N), npt, waves == 8 ? 1 : 2) : form;
 }
 
 extern "C" size_t pq_q8_gemm_workspace_bytes(int N, int K, int T) {
@@ -1068,17 +1095,21 @@ extern "C" int pq_q8_gemm_ws(const int8_t *pcodes, const uint16_t *pscales, cons
   const int form = gemm_form(N, K, T);
   if (form == kFormRows) {
     const int npt = (T + 31) / 32, ngr = (N + kRwRows - 1) / kRwRows;
-    launch(q8_gemm_rows_kernel, dim3((unsigned)((ngr + 7) / 8 * 8 * npt)), dim3(512), kGemmLds, st, pcodes, pscales, qx, dx,
-           y, yb, N, K, T, npt);
+    const int even = group_even(ngr, npt, 1);
+    launch(q8_gemm_rows_kernel, dim3(group_grid(ngr, npt, even)), dim3(512), kGemmLds, st, pcodes, pscales, qx, dx, y, yb, N,
+           K, T, npt, even);
     return check_launch("pq_q8_gemm");
   }
   if (form == kFormChunk) {
     const int npt = (T + 31) / 32;
-    const dim3 grid((unsigned)((ntiles(N) + 7) / 8 * 8 * npt));
-    if (chunk_waves(N, T) == 8)
-      launch(q8_gemm_chunk_kernel<8>, grid, dim3(512), 8 * kCkWave, st, pcodes, pscales, qx, dx, y, yb, N, K, T, npt);
+    const int waves = chunk_waves(N, T), even = group_even(ntiles(N), npt, waves == 8 ? 1 : 2);
+    const dim3 grid(group_grid(ntiles(N), npt, even));
+    if (waves == 8)
+      launch(q8_gemm_chunk_kernel<8>, grid, dim3(512), 8 * kCkWave, st, pcodes, pscales, qx, dx, y, yb, N, K, T, npt,
+             even);
     else
-      launch(q8_gemm_chunk_kernel<4>, grid, dim3(256), 4 * kCkWave, st, pcodes, pscales, qx, dx, y, yb, N, K, T, npt);
+      launch(q8_gemm_chunk_kernel<4>, grid, dim3(256), 4 * kCkWave, st, pcodes, pscales, qx, dx, y, yb, N, K, T, npt,
+             even);
     return check_launch("pq_q8_gemm");
   }
   if (form == kFormSlice) {

@@ -37,12 +37,23 @@ def test_gemm_forms_refuse_what_the_calls_refuse():
     assert L.pq_qlow_gemm_form(64, 2048, 4, 6) == -1 and L.pq_qlow_gemm_form(64, 16640, 4, 4) == -1
 
 
+def test_gemm_even_split_over_xcds():
+    """Whole row groups per XCD must not cost a round of workgroups that the chip as a whole does not need."""
+    form = lib().pq_q8_gemm_form
+    assert form(3104, 2048, 160) == 2 + 16 * 8 + 256    # 49 tiles x 5: 35 workgroups on one XCD's 32 CUs, 245 in all
+    assert form(3104, 2048, 320) == 2 + 16 * 4 + 256    # 490 of 512, 70 of 64
+    assert form(8200, 2048, 384) == 4 + 256             # 17 row groups x 12: 204 of 256, 36 of 32
+    assert form(3104, 2048, 128) == 2 + 16 * 8          # 28 of 32 already
+    assert form(33000, 2048, 256) == 4                  # three rounds either way
+    assert form(16384, 2048, 256) == 4
+
+
 def test_gemm_workspace_only_for_the_walking_form():
     """No other form of the Q8_0 GEMM splits K over workgroups through memory."""
     L = lib()
     for N in (1, 300, 3104, 8000, 16384, 40000):
         for K in (32, 2048, 8192):
             for T in (1, 32, 33, 97, 256):
-                if L.pq_q8_gemm_form(N, K, T) != 1:
+                if L.pq_q8_gemm_form(N, K, T) % 16 != 1:
                     assert L.pq_q8_gemm_workspace_bytes(N, K, T) == 0
     assert L.pq_q8_gemm_form(2048, 8192, 32) == 1 and L.pq_q8_gemm_workspace_bytes(2048, 8192, 32) > 0

@@ -148,10 +148,13 @@ def test_gemm_bitexact(orc, pq, dev, N, K, T):
 @pytest.mark.parametrize("waves,N,K,T", [
     (8, 1, 32, 33), (8, 65, 224, 64), (8, 64, 256, 65), (8, 127, 2080, 100), (8, 300, 4384, 40), (8, 520, 16384, 36),
     (4, 8000, 32, 97), (4, 8000, 288, 97), (4, 4097, 1024, 161), (4, 2112, 2304, 300), (4, 8031, 2272, 97),
-    (4, 4160, 8192, 129)])
+    (4, 4160, 8192, 129),
+    # one XCD would have more row groups than its share of workgroups: an even split
+    (8, 3088, 288, 160), (8, 2100, 2048, 200), (4, 13000, 288, 140)])
 def test_gemm_chunk_form(orc, pq, dev, waves, N, K, T):
     print(f"gemm chunks waves={waves} N={N} K={K} T={T}", flush=True)
-    assert pq.lib().pq_q8_gemm_form(N, K, T) == 2 + 16 * waves
+    even = (N, T) in ((3088, 160), (2100, 200), (13000, 140))
+    assert pq.lib().pq_q8_gemm_form(N, K, T) == 2 + 16 * waves + 256 * even
     W, S, w = _weights(orc, pq, dev, N, K, SEED + 7 * N + K)
     x = orc.gen_normal(SEED + 5 * T + K, T * K).reshape(T, K)
     qx_r, dx_r = orc.q8_quant(x)
@@ -164,10 +167,11 @@ def test_gemm_chunk_form(orc, pq, dev, waves, N, K, T):
 # The row-parallel form (long N): rows that end inside a tile and leave waves of
 # the last group without one, ragged positions, one chunk, one segment of 8 and
 # a ninth chunk in a second.
-@pytest.mark.parametrize("N,K,T", [(15900, 512, 256), (15872, 2304, 250), (16100, 256, 225), (32700, 2048, 128)])
+@pytest.mark.parametrize("N,K,T", [(15900, 512, 256), (15872, 2304, 250), (16100, 256, 225), (32700, 2048, 128),
+                                   (8200, 256, 384), (9000, 512, 353)])
 def test_gemm_row_form(orc, pq, dev, N, K, T):
     print(f"gemm rows N={N} K={K} T={T}", flush=True)
-    assert pq.lib().pq_q8_gemm_form(N, K, T) == 4
+    assert pq.lib().pq_q8_gemm_form(N, K, T) == 4 + 256 * (N < 10000)   # 17 and 18 row groups: an even split
     W, S, w = _weights(orc, pq, dev, N, K, SEED + 3 * N + K)
     x = orc.gen_normal(SEED + 9 * T + K, T * K).reshape(T, K)
     qx_r, dx_r = orc.q8_quant(x)
