@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kRThreads * CW) void q8r_gemv_kc_kernel(const int8_
 // every position runs the leaf chains and the tree of the single-position
 // kernel. The chunk partials of a (position, row) go to an LDS running sum in
 // chunk order, y = ((0 + p_0) + p_1) + ...
-constexpr int kRTPW = 8;       // positions at most
+constexpr int kRTPW = 18;      // positions at most
 
 // RAG: some leaf has fewer than BPL blocks. Its missing ones dot zero codes with
 // block 0's x and are dropped by q8r_leaf's select, which costs 1% where it is
@@ -276,10 +276,29 @@ static int q8r_bpl(int K) { return (q8r_chunk(K) / kQ + 31) / 32; }   // blocks 
 // by the position. Per launch, vector / matrix: 2048 x 2048 at 8 positions 8.3 /
 // 9.0 us, 16384 x 2048 22.5 / 22.3, at 12 positions 512 x 2048 10.6 / 8.6; with
 // over 2 blocks a leaf (codes widened per use, 4.4 us a position at 2048 x 7680)
-// at 4 positions 17.4 / 24.3, at 8 30.9 / 24.7.
+// at 4 positions 17.4 / 24.3, at 8 30.9 / 24.7. From 9 to kRTPW positions in one
+// chunk of K the vector kernel stays where the matrix tiles leave their last
+// round over the CUs mostly empty, by the time of the busiest CU in ns: c
+// workgroups of 8 rows (an odd last one runs beside another), or r tiles, the
+// first in a wave's latency. Fitted to (us, vector / matrix, * the form taken)
+// 4200 x 2048 at 9 9.6* / 11.8, at 13 12.4 / 11.8*; 6144 at 10 10.5* / 12.0, at 13 12.7 /
+// 12.0*; 10000 at 10 14.0* / 15.8, at 12 17.1 / 15.9*, at 17 22.2* / 24.8; 11000 at 9 17.4 /
+// 15.9*; 12300 at 10 19.0* / 19.9; 16384 at 9 21.7 / 20.6*; 17000 at 9 22.4* / 23.8, at 11
+// 25.9 / 24.0*; 20000 x 1024 at 9 13.4* / 17.4; 30000 at 12 23.3 / 22.3*; 9000 x 512 at 9
+// 7.5 / 7.3*.
 static int q8r_form(int N, int K, int T) {
   static const int env_t = env_int("PQ_Q8R_POSWISE");   // 1: one position per workgroup row at any T
-  return env_t != 1 && T > (q8r_bpl(K) <= 2 ? kRTPW : 5) ? q8r_mfma_tile(N, T) : 0;
+  const int bpl = q8r_bpl(K);
+  if (env_t == 1 || T <= (bpl <= 2 ? 8 : 5)) return 0;
+  const int mt = q8r_mfma_tile(N, T);
+  if (T > kRTPW || bpl > 2 || q8r_chunk(K) != K) return mt;
+  const long long c = (N + 2047LL) / 2048, r = ((long long)((N + mt - 1) / mt) * ((T + mt - 1) / mt) + 255) / 256;
+  const long long per = bpl == 1 ? std::max(325LL, 110 * c)
+                                 : std::max(650LL, 250 * c - (c % 2 == 1 ? 212 : c == 4 ? 100 : 0));
+  const long long t_m = mt == 16 ? 2200 + 3150LL * K / 1024 +
+                                       (bpl == 1 && r == 5 ? r : r - 1) * (900 + 1500LL * K / 1024)
+                                 : 2600 + 6350LL * K / 1024 + (r - 1) * (600 + 4600LL * K / 1024);
+  return (4000 + T * per) * 51 / 50 < t_m ? 0 : mt;
 }
 
 extern "C" int pq_q8r_gemv_form(int N, int K, int T) {

@@ -48,6 +48,20 @@ def test_gemm_even_split_over_xcds():
     assert form(16384, 2048, 256) == 4
 
 
+def test_q8r_vector_form_beside_idle_tiles():
+    """9 to 18 positions stay on the vector kernel where 16- or 32-wide tiles give the CUs an almost empty last
+    round (6144 rows: 384 tiles, 10000: 625 16-wide ones, or 313 32-wide)."""
+    form = lib().pq_q8r_gemv_form
+    for N, K, T in ((6144, 2048, 9), (6144, 2048, 10), (10000, 2048, 9), (10000, 2048, 10), (10000, 2048, 17),
+                    (20000, 1024, 9), (8200, 2048, 9)):
+        assert form(N, K, T) == 0, (N, K, T)
+    for N, K, T in ((2048, 2048, 9), (4096, 2048, 9), (6144, 2048, 14), (10000, 2048, 12), (16384, 2048, 9),
+                    (65536, 2048, 9), (16384, 512, 9), (2048, 8192, 9), (2048, 7680, 6), (10000, 2048, 19)):
+        assert form(N, K, T) in (16, 32), (N, K, T)
+    for N in (1, 512, 6144, 65536):
+        assert form(N, 2048, 8) == 0 and form(N, 7680, 5) == 0
+
+
 def test_gemm_workspace_only_for_the_walking_form():
     """No other form of the Q8_0 GEMM splits K over workgroups through memory."""
     L = lib()

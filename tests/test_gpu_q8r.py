@@ -26,9 +26,10 @@ def _run(pq, dev, W, S, xb, dt):
     return y
 
 
-# T = 2 .. 8 (5 with over 2 blocks a leaf) run the T-wide vector form, x staged
-# up to 8 positions at a time: one 2048-wide chunk of 8 positions fills several
-# stagings; more positions run the matrix form. K = 8192 and 12288 fold several
+# T = 2 .. 8 (5 with over 2 blocks a leaf; up to 18 where the matrix tiles would
+# leave most CUs idle: 6150 rows at 10, 9999 at 17) run the T-wide vector form, x
+# staged up to 8 positions at a time: one 2048-wide chunk of 8 positions fills
+# several stagings; more positions run the matrix form. K = 8192 and 12288 fold several
 # 2048-wide chunks, K = 7680 and 2560 are one chunk of 240 and 80 blocks (leaves
 # with several blocks, codes widened per use); at T = 1
 # rows of 2..8 chunks on few workgroups split their chunks over half-waves
@@ -40,11 +41,11 @@ def _run(pq, dev, W, S, xb, dt):
                                    (64, 12288, 5), (45, 2560, 17), (300, 4096, 1), (33, 16384, 1),
                                    (7, 6144, 1), (2048, 7680, 1), (131, 5120, 1), (40, 8160, 1),
                                    (65, 2048, 8), (300, 1024, 8), (33, 6144, 8), (97, 7680, 5), (15, 8160, 4),
-                                   (9, 2080, 5), (12, 96, 8)])
+                                   (9, 2080, 5), (12, 96, 8), (6150, 2048, 10), (9500, 2016, 9), (9999, 2048, 17)])
 def test_q8r_gemv_bitexact(orc, pq, dev, N, K, T):
     print(f"q8r N={N} K={K} T={T}", flush=True)
     W, S, xb = _case(orc, N, K, T, SEED + N + K, signed_scales=(N % 2 == 1))
-    assert (pq.lib().pq_q8r_gemv_form(N, K, T) == 0) == (T <= (8 if K <= 2048 or K % 2048 == 0 else 5))
+    assert pq.lib().pq_q8r_gemv_form(N, K, T) == 0 or T > (8 if K <= 2048 or K % 2048 == 0 else 5)
     want = orc.q8r_gemm(W, S, xb)
     y = _run(pq, dev, W, S, xb, pq.DT_F32).cpu().numpy()
     assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
